@@ -450,7 +450,7 @@ gtd::DScene device_scene(const gt_scene* s, uint32_t width) {
 
 uint64_t stack_depth(const gt_scene* s, uint32_t width) {
   uint64_t d = width == 4 ? s->packed.depth4 * 3 : s->packed.depth2;  // wide nodes push up to 3 per level
-  return d + 2;
+  return d + 3;  // one entry ends a walk
 }
 
 // LDS traversal-stack entries per lane (gt_tuning.stack_lds); 8 measured
@@ -460,14 +460,25 @@ uint32_t stack_cap(const gt_context* ctx) {
   return ctx->tuning.stack_lds ? ctx->tuning.stack_lds : kDefaultStackLds;
 }
 
+// When the traversal kernels top a wave up with new rays (Queues::refill_at).
+// Walks of the smallest trees are a few steps, about equally many for every
+// ray: refilling a wave costs more than its idle lanes. On one MI355X, without
+// and with refill: 15 nodes (Cornell box 512^2, 32 spp) 6.56 and 6.86 ms; 65
+// nodes (129 spheres, 960x540, 16 spp) 1.74 and 1.70 ms; 465 nodes 3.86 and
+// 3.74 ms; 2695 nodes 3.55 and 3.30 ms. Refilling at 24 lanes against 32 and 40:
+// terrain 720p 13.7, 13.9 and 14.0 ms; 1080p GGX/environment 13.1, 13.2 and 13.6 ms.
+constexpr uint64_t kRefillNodes = 32;
+constexpr uint32_t kRefillAt = 24;
+
 // Persistent grid: blocks_per_cu per CU, or as many as the occupancy of the
 // traversal kernels allows (their LDS stack is the binding limit).
 uint32_t grid_for(gt_context* ctx) {
   uint32_t bpc = ctx->tuning.blocks_per_cu;
   if (bpc == 0) {
     uint32_t b = ctx->tuning.block_size;
-    size_t lds = gtk::stack_lds_bytes(b, stack_cap(ctx));
-    bpc = std::max<uint32_t>(1, std::min(gtk::occupancy_blocks(0, b, lds), gtk::occupancy_blocks(2, b, lds)));
+    const uint32_t cap = stack_cap(ctx);
+    bpc = std::max<uint32_t>(1, std::min(gtk::occupancy_blocks(0, b, gtk::extend_lds_bytes(b, cap)),
+                                         gtk::occupancy_blocks(2, b, gtk::stack_lds_bytes(b, cap))));
   }
   return std::max<uint32_t>(1, ctx->cus * bpc);
 }
@@ -517,6 +528,7 @@ gtk::Queues queues_of(gt_context* ctx) {
   q.gstack = ctx->gstack.p;
   q.gstride = ctx->gstride;
   q.stack_cap = stack_cap(ctx);
+  q.refill_at = 0;  // run_jobs decides
   return q;
 }
 
@@ -579,6 +591,7 @@ struct FrameJob {
   const gtk::Adapt* adapt = nullptr;    // adaptive round: Welford update instead of accumulation
   bool conn_l = false, conn_e = false;  // light / environment shadow rays
   uint64_t stack_need = 0;
+  uint64_t nodes = 0;                   // inner nodes of the scene's binary tree
   void* d_out = nullptr;                // finalize target (float or double W*H*3), or null
 };
 
@@ -636,7 +649,7 @@ int run_jobs(gt_context* ctx, std::vector<FrameJob>& jobs, bool multi, int out_i
   uint64_t cap = max_paths_override ? max_paths_override
                                     : (ctx->tuning.max_paths ? ctx->tuning.max_paths : (uint64_t(1) << 25));
   cap = std::min<uint64_t>(cap, uint64_t(1) << 31);
-  uint64_t acc_total = 0, stack_need = 0;
+  uint64_t acc_total = 0, stack_need = 0, nodes = 0;
   uint32_t depth_all = 0;
   const bool adaptive = !multi && jobs.size() == 1 && jobs[0].adapt != nullptr;
   for (FrameJob& j : jobs) {
@@ -646,6 +659,7 @@ int run_jobs(gt_context* ctx, std::vector<FrameJob>& jobs, bool multi, int out_i
     acc_total += j.f.npix;
     depth_all = std::max(depth_all, j.depth);
     stack_need = std::max(stack_need, j.stack_need);
+    nodes = std::max(nodes, j.nodes);
   }
   if (acc_total >= (uint64_t(1) << 31)) return fail(GT_EINVAL, "batch too large (2^31 pixels in total)");
   std::vector<std::vector<gtk::Seg>> batches = plan_batches(jobs, cap, !multi);
@@ -680,6 +694,7 @@ int run_jobs(gt_context* ctx, std::vector<FrameJob>& jobs, bool multi, int out_i
     GT_HIP(hipStreamSynchronize(ctx->stream));  // the host tables go out of scope
   }
   gtk::Queues q = queues_of(ctx);
+  q.refill_at = nodes >= kRefillNodes ? kRefillAt : 0;
   gtk::Launch L{grid_for(ctx), ctx->tuning.block_size, ctx->stream};
   hipStream_t st = ctx->stream;
   const size_t nbatch = batches.size();
@@ -721,6 +736,7 @@ int run_jobs(gt_context* ctx, std::vector<FrameJob>& jobs, bool multi, int out_i
     for (size_t b = 0; b < nbatch; ++b) {
       gtk::Work w{};
       w.multi = multi;
+      w.wide = ctx->tuning.bvh_width == 4;
       w.bt.nseg = uint32_t(batches[b].size());
       uint64_t total = 0, pix = 0;
       for (auto& sg : batches[b]) {
@@ -877,6 +893,7 @@ int prepare_job(gt_context* ctx, const gt_scene* cscene, const gt_camera* camera
   j->conn_l = j->f.nee && lights != nullptr;
   j->conn_e = j->f.nee && env != nullptr;
   j->stack_need = stack_depth(scene, j->f.scene.width);
+  j->nodes = scene->n_nodes2;
   return GT_OK;
 }
 

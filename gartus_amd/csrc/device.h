@@ -49,6 +49,17 @@ __device__ __forceinline__ bool finite3(f3 a) { return isfinite(a.x) && isfinite
 __device__ __forceinline__ float clampf(float x, float lo, float hi) { return x < lo ? lo : (x > hi ? hi : x); }
 __device__ __forceinline__ float pow5(float x) { float x2 = x * x; float x4 = x2 * x2; return x * x4; }
 __device__ __forceinline__ f3 ld3(const float* p) { return {p[0], p[1], p[2]}; }
+// A table in device memory that no kernel writes, at a wave-uniform address,
+// as constant memory: its fields load as scalars, and the compiler takes the
+// pointers among them for global ones. (Through generic pointers it would use
+// flat instructions, which also occupy the LDS path and its wait counter.)
+template <class T>
+__device__ __forceinline__ const T& as_constant(const T* p) {
+  typedef const __attribute__((address_space(4))) T* P;
+  const uint64_t a = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(a)), hi = __builtin_amdgcn_readfirstlane(uint32_t(a >> 32));
+  return *(const T*)(P)(uint64_t(hi) << 32 | lo);
+}
 
 // ---- RNG: SplitMix64 (random.rs:23-29) -------------------------------------
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
@@ -466,8 +477,9 @@ __device__ __forceinline__ f3 prim_outward_normal(const GPrim* __restrict__ prim
 // flat triangle, any other primitive, or a degenerate interpolation.
 __device__ __forceinline__ f3 shading_normal(const GPrim* __restrict__ prims, const float4* __restrict__ vn,
                                              uint32_t k, float u, float v, bool front, f3 n) {
-  const float4 p1 = reinterpret_cast<const float4*>(prims + k)[1];
-  const uint32_t kind = (meta_of(reinterpret_cast<const float4*>(prims + k)[0]) >> GT_KIND_SHIFT) & GT_KIND_MASK;
+  const float4* rec = reinterpret_cast<const float4*>(prims + k);
+  const float4 p1 = rec[1];
+  const uint32_t kind = (meta_of(rec[0]) >> GT_KIND_SHIFT) & GT_KIND_MASK;
   const uint32_t smooth = __float_as_uint(p1.w);
   if (kind != GK_TRIANGLE || smooth == 0u) return n;
   const float4* q = vn + 3 * size_t(smooth - 1u);
@@ -510,23 +522,42 @@ struct Stats {
 };
 
 // Per-lane traversal stack: the first `cap` entries in LDS (lane-interleaved),
-// the rest in a per-lane slice of global memory.
+// the rest in a per-lane slice of global memory. Each part is reached through a
+// pointer of its own address space: through a common one the compiler merges
+// the two accesses into flat instructions, which occupy the vector memory path
+// and both wait counters for what is nearly always an LDS access.
+typedef uint32_t stack_entry __attribute__((ext_vector_type(2)));  // child reference, entry distance
+typedef __attribute__((address_space(3))) stack_entry lds_entry;
+typedef __attribute__((address_space(1))) stack_entry global_entry;
 struct Stack {
-  uint2* lds;
-  uint32_t stride;
-  uint2* glob;
+  uint32_t lds;     // LDS address of the lane's first entry
+  uint32_t stride;  // bytes between a lane's entries
+  global_entry* glob;
   uint32_t gstride;
   int cap;
   int n;
+  __device__ __forceinline__ lds_entry* slot() const { return (lds_entry*)(__umul24(n, stride) + lds); }
+  __device__ __forceinline__ global_entry* spill() const { return glob + size_t(uint32_t(n - cap)) * gstride; }
   __device__ __forceinline__ void push(uint32_t ref, float t) {
-    uint2 e = make_uint2(ref, __float_as_uint(t));
-    if (n < cap) lds[n * stride] = e;
-    else glob[size_t(n - cap) * gstride] = e;
+    const stack_entry e = {ref, __float_as_uint(t)};
+    if (__ballot(n >= cap) == 0ull) {  // the usual case for every lane
+      *slot() = e;
+    } else {
+      if (n < cap) *slot() = e;
+      else *spill() = e;
+    }
     ++n;
   }
   __device__ __forceinline__ uint2 pop() {
     --n;
-    return n < cap ? lds[n * stride] : glob[size_t(n - cap) * gstride];
+    stack_entry e;
+    if (__ballot(n >= cap) == 0ull) {
+      e = *slot();
+    } else {
+      if (n < cap) e = *slot();
+      else e = *spill();
+    }
+    return make_uint2(e.x, e.y);
   }
 };
 
@@ -565,12 +596,11 @@ __device__ __forceinline__ bool slab(const RayPre& r, float lox, float hix, floa
   return ex * 1.0000004f >= en;
 }
 
-// Closest hit (ANY = false) or any hit (ANY = true) over the BVH2 layout,
-// walking the reference's order: both children tested against the current
+// Closest hit over the BVH2 layout, walking the reference's order: both children tested against the current
 // closest, nearer first (left on ties), entries pruned when entry >= closest
 // (bvh.rs:306-399). Leaves test primitives in permutation order with the
 // interval shrinking on each accepted hit (scene.rs:849-874).
-template <bool ANY, bool STATS>
+template <bool STATS>
 __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax,
                                        uint32_t self, Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out,
                                        Stats* stats, uint32_t* meta_out = nullptr) {
@@ -587,80 +617,6 @@ __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time,
   if (STATS) { stats->node_hits += 1; stats->max_stack = max(stats->max_stack, 1u); }
   uint32_t cur = sc.root_ref;
   st.n = 0;
-  if (ANY && !STATS) {
-    // Any-hit rays walk while-while with speculation (Aila and Laine,
-    // "Understanding the efficiency of ray traversal on GPUs", HPG 2009): a
-    // ray that reaches a leaf parks it and walks on through inner nodes until
-    // every ray of the wave has a leaf parked, then the wave tests leaves
-    // together. An any-hit query never narrows its interval before it
-    // returns, so it visits the same nodes in either loop and its answer is
-    // the same. (For closest hits the walk would cull with a stale closest hit
-    // and could reach leaves that the reference's pruning skips.)
-    constexpr uint32_t kNone = 0xffffffffu;  // no node: has the leaf bit, so it ends the inner loop
-    uint32_t leaf = kNone;
-    if (cur & GT_LEAF_BIT) { leaf = cur; cur = kNone; }
-    auto next = [&]() -> uint32_t {  // pop, skipping entries that cannot beat the closest hit
-      while (st.n > 0) {
-        const uint2 e = st.pop();
-        if (__uint_as_float(e.y) < closest) return e.x;
-      }
-      return kNone;
-    };
-    while (cur != kNone || leaf != kNone) {
-      while (!(cur & GT_LEAF_BIT)) {
-        const float4* nd = reinterpret_cast<const float4*>(sc.nodes2 + cur);
-        const float4 a = nd[0], b = nd[1], c = nd[2];
-        const uint4 refs = *reinterpret_cast<const uint4*>(nd + 3);
-        float le, re;
-        const bool lh = slab(rp, a.x, a.y, a.z, a.w, c.x, c.y, tmin, closest, &le);
-        const bool rh = slab(rp, b.x, b.y, b.z, b.w, c.z, c.w, tmin, closest, &re);
-        if (lh && rh) {
-          const bool right_first = re < le;
-          st.push(right_first ? refs.x : refs.y, right_first ? le : re);
-          cur = right_first ? refs.y : refs.x;
-        } else if (lh) {
-          cur = refs.x;
-        } else if (rh) {
-          cur = refs.y;
-        } else {
-          cur = next();
-        }
-        if (cur != kNone && (cur & GT_LEAF_BIT) && leaf == kNone) {
-          leaf = cur;
-          cur = next();
-        }
-        if (!__any(leaf == kNone)) break;  // every ray still walking has a leaf parked
-      }
-      while (leaf != kNone) {
-        for (uint32_t k = leaf & ~GT_LEAF_BIT;; ++k) {
-          PrimHit h;
-          uint32_t meta;
-          if (prim_test(sc.prims, k, o, d, time, tmin, closest, &h, &meta, k == self)) {
-            closest = h.t;
-            best = k;
-            best_meta = meta;
-            bh = h;
-            any = true;
-            if (ANY) return true;
-          }
-          if (meta & GT_LAST_BIT) break;
-        }
-        if (cur != kNone && (cur & GT_LEAF_BIT)) {
-          leaf = cur;
-          cur = next();
-        } else {
-          leaf = kNone;
-        }
-      }
-    }
-    if (any) {
-      *t_out = closest;
-      *prim_out = best;
-      if (hit_out) *hit_out = bh;
-      if (meta_out) *meta_out = best_meta;
-    }
-    return any;
-  }
   for (;;) {
     if (cur & GT_LEAF_BIT) {
       uint32_t k = cur & ~GT_LEAF_BIT;
@@ -677,7 +633,6 @@ __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time,
           bh = h;
           any = true;
           leaf_hit = true;
-          if (ANY) return true;
         }
         if (meta & GT_LAST_BIT) break;
         ++k;
@@ -728,7 +683,7 @@ __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time,
 }
 
 // Four-wide variant: children of a wide node are visited nearest-first.
-template <bool ANY, bool STATS>
+template <bool STATS>
 __device__ __forceinline__ bool trace4(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax,
                                        uint32_t self, Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out,
                                        Stats* stats, uint32_t* meta_out = nullptr) {
@@ -756,7 +711,6 @@ __device__ __forceinline__ bool trace4(const DScene& sc, f3 o, f3 d, float time,
         if (STATS) stats->candidates += 1;
         if (prim_test(sc.prims, k, o, d, time, tmin, closest, &h, &meta, k == self)) {
           closest = h.t; best = k; best_meta = meta; bh = h; any = true; leaf_hit = true;
-          if (ANY) return true;
         }
         if (meta & GT_LAST_BIT) break;
         ++k;
@@ -817,13 +771,129 @@ __device__ __forceinline__ bool trace4(const DScene& sc, f3 o, f3 d, float time,
 // self: the primitive (leaf order) the ray starts on, kNoSelf for a ray from
 // a camera or a caller; prim_test decides it by rule, not by t_min.
 constexpr uint32_t kNoSelf = 0xffffffffu;
-template <bool ANY, bool STATS>
+template <bool STATS>
 __device__ __forceinline__ bool trace(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax, uint32_t self,
                                       Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out, Stats* stats,
                                       uint32_t* meta_out = nullptr) {
   if (sc.width == 4)
-    return trace4<ANY, STATS>(sc, o, d, time, tmin, tmax, self, st, t_out, prim_out, hit_out, stats, meta_out);
-  return trace2<ANY, STATS>(sc, o, d, time, tmin, tmax, self, st, t_out, prim_out, hit_out, stats, meta_out);
+    return trace4<STATS>(sc, o, d, time, tmin, tmax, self, st, t_out, prim_out, hit_out, stats, meta_out);
+  return trace2<STATS>(sc, o, d, time, tmin, tmax, self, st, t_out, prim_out, hit_out, stats, meta_out);
+}
+
+// ---- resumable walk -----------------------------------------------------------
+// The same search as trace, one step at a time: the state of a ray between
+// steps, so that a wave can mix rays at different points of their walks. A
+// ray's steps (nodes fetched, primitives tested, the closest hit each is tested
+// against) are those of trace2 / trace4, in the same order, whatever the other
+// lanes do. tmin is SHADOW_ACNE and the interval starts unbounded.
+constexpr uint32_t kNoNode = 0xffffffffu;  // walk over (has the leaf bit; no leaf has this index)
+constexpr uint32_t kNoPrim = 0xffffffffu;
+struct Walk {
+  f3 o, d;
+  float inv[3];
+  float time, closest;
+  uint32_t cur;  // node, GT_LEAF_BIT | primitive, or kNoNode
+  uint32_t self, best;
+};
+// The scene's part that the steps read, with pointers known to be global.
+struct WalkScene {
+  const float4* nodes;  // GNode2 or GNode4 records
+  const GPrim* prims;
+};
+template <bool WIDE>
+__device__ __forceinline__ WalkScene walk_scene(const DScene& sc) {
+  return {WIDE ? reinterpret_cast<const float4*>(sc.nodes4) : reinterpret_cast<const float4*>(sc.nodes2),
+          sc.prims};
+}
+// The stack's bottom entry ends the walk, so a pop needs no test for an empty stack.
+__device__ __forceinline__ void walk_begin(const DScene& sc, f3 o, f3 d, float time, uint32_t self, Walk& w, Stack& st) {
+  const RayPre rp = ray_pre(o, d);
+  w.o = o;
+  w.d = d;
+  for (int a = 0; a < 3; ++a) w.inv[a] = rp.inv[a];
+  w.time = time;
+  w.closest = INF;
+  w.self = self;
+  w.best = kNoPrim;
+  st.n = 0;
+  st.push(kNoNode, -INF);
+  float entry;
+  w.cur = slab(rp, sc.root_lo[0], sc.root_hi[0], sc.root_lo[1], sc.root_hi[1], sc.root_lo[2], sc.root_hi[2],
+               SHADOW_ACNE, INF, &entry)
+              ? sc.root_ref
+              : kNoNode;
+}
+// The next stack entry that can beat the closest hit, or kNoNode.
+__device__ __forceinline__ uint32_t walk_pop(float closest, Stack& st) {
+  uint2 e;
+  do e = st.pop();
+  while (!(__uint_as_float(e.y) < closest));
+  return e.x;
+}
+// One inner node: w.cur is a node index.
+template <bool WIDE>
+__device__ __forceinline__ void walk_inner(const WalkScene& sc, Walk& w, Stack& st) {
+  RayPre rp;
+  rp.o = w.o;
+  for (int a = 0; a < 3; ++a) { rp.inv[a] = w.inv[a]; rp.neg[a] = w.inv[a] < 0.f; }
+  if (!WIDE) {
+    const float4* nd = sc.nodes + 4 * size_t(w.cur);
+    const float4 a = nd[0], b = nd[1], c = nd[2];
+    const uint2 refs = *reinterpret_cast<const uint2*>(nd + 3);
+    float le, re;
+    const bool lh = slab(rp, a.x, a.y, a.z, a.w, c.x, c.y, SHADOW_ACNE, w.closest, &le);
+    const bool rh = slab(rp, b.x, b.y, b.z, b.w, c.z, c.w, SHADOW_ACNE, w.closest, &re);
+    const bool nearer = re < le;
+    const bool right = lh ? nearer : true;  // the nearer child, left on ties
+    const bool r = rh ? right : false;
+    const bool both = lh ? rh : false, none = lh ? false : !rh;
+    w.cur = r ? refs.y : refs.x;
+    if (both) st.push(r ? refs.x : refs.y, r ? le : re);
+    if (none) w.cur = walk_pop(w.closest, st);
+    return;
+  }
+  const float4* nd = sc.nodes + 8 * size_t(w.cur);
+  const float4 lox = nd[0], hix = nd[1], loy = nd[2], hiy = nd[3], loz = nd[4], hiz = nd[5];
+  const uint4 ch = *reinterpret_cast<const uint4*>(nd + 6);
+  float e[4];
+  bool h[4];
+  h[0] = slab(rp, lox.x, hix.x, loy.x, hiy.x, loz.x, hiz.x, SHADOW_ACNE, w.closest, &e[0]) && ch.x != GT_EMPTY_CHILD;
+  h[1] = slab(rp, lox.y, hix.y, loy.y, hiy.y, loz.y, hiz.y, SHADOW_ACNE, w.closest, &e[1]) && ch.y != GT_EMPTY_CHILD;
+  h[2] = slab(rp, lox.z, hix.z, loy.z, hiy.z, loz.z, hiz.z, SHADOW_ACNE, w.closest, &e[2]) && ch.z != GT_EMPTY_CHILD;
+  h[3] = slab(rp, lox.w, hix.w, loy.w, hiy.w, loz.w, hiz.w, SHADOW_ACNE, w.closest, &e[3]) && ch.w != GT_EMPTY_CHILD;
+  const uint32_t c[4] = {ch.x, ch.y, ch.z, ch.w};
+  // as trace4: hit children by entry (lower slot first on ties), all but the nearest pushed far to near
+  int idx[4];
+  int nh = 0;
+  for (int k = 0; k < 4; ++k) if (h[k]) idx[nh++] = k;
+  for (int i = 1; i < nh; ++i) {
+    int v = idx[i];
+    int j = i - 1;
+    while (j >= 0 && e[idx[j]] > e[v]) { idx[j + 1] = idx[j]; --j; }
+    idx[j + 1] = v;
+  }
+  if (nh > 0) {
+    for (int i = nh - 1; i >= 1; --i) st.push(c[idx[i]], e[idx[i]]);
+    w.cur = c[idx[0]];
+  } else {
+    w.cur = walk_pop(w.closest, st);
+  }
+}
+// One primitive of a leaf: w.cur is GT_LEAF_BIT | its index. With ANY the first hit ends the walk.
+template <bool ANY>
+__device__ __forceinline__ void walk_leaf(const WalkScene& sc, Walk& w, Stack& st) {
+  const uint32_t k = w.cur & ~GT_LEAF_BIT;
+  PrimHit h;
+  uint32_t meta;
+  bool over = false;
+  if (prim_test(sc.prims, k, w.o, w.d, w.time, SHADOW_ACNE, w.closest, &h, &meta, k == w.self)) {
+    w.closest = h.t;
+    w.best = k;
+    over = ANY;
+  }
+  w.cur += 1;
+  if (over) w.cur = kNoNode;
+  else if (meta & GT_LAST_BIT) w.cur = walk_pop(w.closest, st);
 }
 
 // ---- light targets (scene.rs:363-609, object.rs:1048-1161) --------------------
@@ -992,8 +1062,9 @@ __device__ __forceinline__ f3 env_radiance_uv(const DEnv& e, float u, float v) {
   uint32_t y0 = min(uint32_t(floorf(cy)), e.h - 1);
   uint32_t y1 = min(y0 + 1, e.h - 1);
   float tx = cx - float(x0), ty = cy - float(y0);
-  float4 a = e.tex[size_t(y0) * e.w + x0], b = e.tex[size_t(y0) * e.w + x1];
-  float4 c = e.tex[size_t(y1) * e.w + x0], f = e.tex[size_t(y1) * e.w + x1];
+  const float4* tex = e.tex;
+  float4 a = tex[size_t(y0) * e.w + x0], b = tex[size_t(y0) * e.w + x1];
+  float4 c = tex[size_t(y1) * e.w + x0], f = tex[size_t(y1) * e.w + x1];
   f3 top = mk(a.x + (b.x - a.x) * tx, a.y + (b.y - a.y) * tx, a.z + (b.z - a.z) * tx);
   f3 bot = mk(c.x + (f.x - c.x) * tx, c.y + (f.y - c.y) * tx, c.z + (f.z - c.z) * tx);
   return top + (bot - top) * ty;

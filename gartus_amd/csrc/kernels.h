@@ -65,6 +65,7 @@ struct Queues {
   uint2* gstack;    // traversal-stack overflow, gstride entries per level
   uint32_t gstride;
   uint32_t stack_cap;  // LDS entries per lane
+  uint32_t refill_at;  // a traversal wave takes new rays when at most this many lanes still walk
 };
 
 // Everything one render of one scene reads: scene, lights, environment,
@@ -126,6 +127,7 @@ struct Work {
   Frame f;
   Batch bt;
   bool multi;
+  bool wide;  // the frames' inner nodes are four-wide
 };
 
 void reset_counters(const Launch& l, const Queues& q, uint32_t depth, uint32_t total);
@@ -177,5 +179,8 @@ uint32_t occupancy_blocks(int kernel, uint32_t block, size_t lds_bytes);
 
 // Bytes of LDS per block for the traversal stack.
 inline size_t stack_lds_bytes(uint32_t block, uint32_t cap) { return size_t(block) * cap * sizeof(uint2); }
+
+// ... of an extend block: the stack and the waves' rings of finished paths.
+size_t extend_lds_bytes(uint32_t block, uint32_t cap);
 
 }  // namespace gtk

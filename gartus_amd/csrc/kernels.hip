@@ -77,9 +77,9 @@ __device__ __forceinline__ void wave_append_chunk(uint32_t* counter, uint32_t* l
 
 __device__ __forceinline__ Stack make_stack(const Queues& q, uint2* smem) {
   Stack st;
-  st.lds = smem + threadIdx.x;
-  st.stride = blockDim.x;
-  st.glob = q.gstack + (blockIdx.x * blockDim.x + threadIdx.x);
+  st.lds = uint32_t(reinterpret_cast<uintptr_t>((lds_entry*)(smem + threadIdx.x)));
+  st.stride = blockDim.x * uint32_t(sizeof(stack_entry));
+  st.glob = (global_entry*)(q.gstack + (blockIdx.x * blockDim.x + threadIdx.x));
   st.gstride = q.gstride;
   st.cap = int(q.stack_cap);
   st.n = 0;
@@ -129,7 +129,7 @@ __device__ __forceinline__ void with_frame(const Frame& f0, const Batch& bt, boo
         const uint32_t u = __builtin_amdgcn_readfirstlane(mine);
         if (mine == u) {
           const Seg sg = bt.segs[u];
-          body(bt.frames[sg.frame], sg);
+          body(as_constant(bt.frames + sg.frame), sg);
           pending = false;
         }
       }
@@ -227,13 +227,7 @@ __device__ __forceinline__ uint32_t node_fetches(const Stats& s, uint32_t width)
   return (s.node_tests - 1) / width;
 }
 
-// Camera rays for samples [sample0, sample0 + nsamples) of every pixel
-// (render_world_linear_pixel_with_context camera.rs:2660-2723; rays :1658-1718).
-// Closest hit of every active path; each hit is binned by the shading
-// category of its material; a miss is shaded on the spot. At bounce 0
-// (CAMERA) the kernel generates the camera rays itself (camera.rs:1658-1718)
-// and stores a path's state only if it hit something: a path that misses
-// ends here with the background as its radiance.
+// Shading category of a primitive's material.
 __device__ __forceinline__ uint32_t category_of(uint32_t meta) {
   switch ((meta >> GT_MATKIND_SHIFT) & 7u) {
     case GM_DIFFUSE_LIGHT: return CAT_EMIT;
@@ -245,92 +239,252 @@ __device__ __forceinline__ uint32_t category_of(uint32_t meta) {
   }
 }
 
-template <bool COUNT, bool MULTI, bool CAMERA>
+// ---- traversal with refill ---------------------------------------------------
+// What bounds the traversal kernels is the vector ALU: before, its instructions
+// filled 70 to 98 % of a SIMD's cycles on the 1080p GGX/environment frame and
+// the 720p terrain, with 21 to 40 % of their lanes at work, because the rays of
+// a wave differ widely in length and wait for the longest. So the walk of
+// every lane is resumable (Walk), a wave takes new rays whenever at most
+// refill_at lanes still walk, and finished lanes are retired at the same point,
+// together. A step serves either the lanes at an inner node or those at a
+// primitive, whichever are more. The steps run in a loop of their own, whose
+// carried state is only what a step changes (carrying the whole ray around one
+// common loop cost 32 moves a step); everything else is read from the kernel's
+// arguments when it is needed. Measured against one ray per lane at a time, on
+// one MI355X: 720p terrain 16.2 -> 13.7 ms, 1080p GGX/environment 14.4 -> 13.1 ms,
+// 12 small scenes in one batch 8.3 -> 5.3 ms (also for the scene pointers no
+// longer being generic, whose loads were flat instructions). Camera rays are
+// coherent and as long as their neighbours: they take no refill.
+constexpr uint32_t kRing = 128;                   // entries of a wave's ring: at most 63 + 64 are held
+constexpr uint32_t kRingWords = 2 * kRing;        // extend: finished hits, finished misses
+constexpr uint32_t kNoPath = 0xffffffffu;
+
+// The arguments of a traversal kernel, read where they are needed: the address
+// is hidden from the compiler, which otherwise loads all of them up front and
+// spills them to vector registers around the walk.
+struct Args {
+  Frame f;
+  Batch bt;
+  Queues q;
+  uint32_t bounce;
+};
+__device__ __forceinline__ const Args& kernel_args() {
+  typedef const __attribute__((address_space(4))) Args* P;
+  P p = (P)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Args*)p;
+}
+
+__device__ __forceinline__ uint32_t count_lanes(bool b) { return uint32_t(__popcll(__ballot(b))); }
+__device__ __forceinline__ uint32_t rank_below(unsigned long long mask) {
+  return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0u));
+}
+
+// A wave's claim on a slice's queue: entries [lo, hi) are claimed and not yet taken.
+struct Claim {
+  uint32_t lo = 0, hi = 0;
+  bool more = true;
+  // Hands every lane with want set the next entry (its index in *j) while there are any;
+  // returns whether this lane got one.
+  __device__ __forceinline__ bool take(uint32_t* cursor, uint32_t per_lane, uint32_t count, bool want, uint32_t* j) {
+    bool got = false;
+    for (;;) {
+      const unsigned long long need = __ballot(want && !got);
+      if (need == 0ull) break;
+      if (lo == hi) {
+        if (!more) break;
+        const uint32_t base = __builtin_amdgcn_readfirstlane(wave_fetch(cursor, per_lane));
+        if (base >= count) {
+          more = false;
+          break;
+        }
+        lo = base;
+        hi = min(base + per_lane * 64u, count);
+      }
+      const uint32_t n = min(uint32_t(__popcll(need)), hi - lo), r = rank_below(need);
+      if (want && !got && r < n) {
+        *j = lo + r;
+        got = true;
+      }
+      lo += n;
+    }
+    return got;
+  }
+  __device__ __forceinline__ bool left() const { return more || lo != hi; }
+};
+
+// The walk of a wave over one slice's queue. POLICY supplies:
+//   entry(j)                     path of queue entry j
+//   start(a, f, sg, p, w, st)    loads or makes path p's ray and begins its walk (false: nothing to trace)
+//   retire(a, fin, p, w)         called with every lane; fin marks the lanes whose walk just ended
+// In a batched render the lanes of a wave may walk different scenes.
+template <bool MULTI, bool WIDE, bool ANY, bool COUNT, class POLICY>
+__device__ __forceinline__ void walk_queue(Stack& st, uint32_t* cursor, uint32_t count, uint32_t refill_at, POLICY&& pol,
+                                           uint32_t& nodes, uint32_t& prims) {
+  const uint32_t per_lane = items_per_lane(count);
+  Claim claim;
+  Walk w;
+  w.cur = kNoNode;
+  uint32_t p = kNoPath;  // the path a lane walks
+  WalkScene sc = walk_scene<WIDE>(kernel_args().f.scene);
+  for (;;) {
+    {
+      const Args& a = kernel_args();
+      pol.retire(a, p != kNoPath && w.cur == kNoNode, p, w, sc);
+      if (w.cur == kNoNode) p = kNoPath;
+      uint32_t j = 0;
+      const bool go = claim.take(cursor, per_lane, count, p == kNoPath, &j);
+      if (go) p = pol.entry(a, j);
+      with_frame<MULTI>(a.f, a.bt, go, p, [&](const Frame& f, const Seg& sg) {
+        if (MULTI) sc = walk_scene<WIDE>(f.scene);
+        if (!pol.start(a, f, sg, p, w, st)) p = kNoPath;
+      });
+      if (__ballot(p != kNoPath) == 0ull && !claim.left()) break;
+    }
+    // a loop of its own: only what a step changes is carried around it
+    const uint32_t limit = claim.left() ? refill_at : 0u;
+    for (;;) {
+      const uint32_t busy = count_lanes(w.cur != kNoNode);
+      if (busy <= limit) break;
+      const uint32_t ni = count_lanes(int32_t(w.cur) >= 0);
+      if (2 * ni >= busy) {
+        if (int32_t(w.cur) >= 0) {
+          walk_inner<WIDE>(sc, w, st);
+          if (COUNT) ++nodes;
+        }
+      } else if (int32_t(w.cur) < -1) {
+        walk_leaf<ANY>(sc, w, st);
+        if (COUNT) ++prims;
+      }
+    }
+  }
+}
+
+// Closest hit of every active path; each hit is binned by the shading
+// category of its material; a miss is shaded on the spot. At bounce 0
+// (CAMERA) the kernel generates the camera rays itself (camera.rs:1658-1718)
+// and stores a path's state only if it hit something: a path that misses
+// ends here with the background as its radiance.
+template <bool MULTI, bool CAMERA>
+struct ExtendPolicy {
+  uint32_t s, first;              // slice, and its first path: every path of it lies in [first, first + region]
+  uint32_t *ring_hit, *ring_miss;
+  uint32_t nhit = 0, hit0 = 0, nmiss = 0, miss0 = 0;  // ring entries and the oldest one's slot
+
+  // The n oldest finished hits, binned by category with one atomic per category.
+  __device__ __forceinline__ void flush_hits(const Args& a, uint32_t n) {
+    uint32_t e = 0;
+    const bool valid = lane_id() < n;
+    if (valid) e = ring_hit[(hit0 + lane_id()) % kRing];
+    const uint32_t cat = valid ? e >> 29 : uint32_t(kNumCategories);
+#pragma unroll
+    for (uint32_t c = CAT_EMIT; c < kNumCategories; ++c) {
+      const unsigned long long m = __ballot(cat == c);
+      if (m == 0ull) continue;
+      uint32_t base = 0;
+      if (lane_id() == 0)
+        base = atomicAdd(a.q.ctr + ctr_at(a.bounce, S_CAT_COUNT + c, s), uint32_t(__popcll(m)));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (cat == c) (a.q.cat[c] + size_t(s) * a.q.region)[base + rank_below(m)] = first + (e & 0x1fffffffu);
+    }
+    hit0 += n;
+    nhit -= n;
+  }
+  // The n oldest misses end here (camera.rs:1747-1750): background or environment, times the
+  // MIS weight; shading them in place saves a queue and a launch per bounce.
+  __device__ __forceinline__ void flush_misses(const Args& a, uint32_t n) {
+    const bool valid = lane_id() < n;
+    uint32_t p = 0;
+    if (valid) p = ring_miss[(miss0 + lane_id()) % kRing];
+    float4* const radiance = a.q.radiance;
+    with_frame<MULTI>(a.f, a.bt, valid, p, [&](const Frame& f, const Seg&) {
+      const float4 d4 = a.q.ray_d[p];
+      const float4 t4 = CAMERA ? make_float4(1.f, 1.f, 1.f, 1.f) : a.q.thr[p];
+      const f3 d = mk(d4.x, d4.y, d4.z);
+      float mw = t4.w;
+      const f3 rad = f.env.kind != 0 ? env_radiance_weighted(f.env, d, &mw) : background(f.cam, d);
+      const f3 miss = rad * mw;
+      const float4 L = CAMERA ? make_float4(0.f, 0.f, 0.f, 0.f) : radiance[p];
+      radiance[p] = make_float4(L.x + t4.x * miss.x, L.y + t4.y * miss.y, L.z + t4.z * miss.z, 0.f);
+    });
+    miss0 += n;
+    nmiss -= n;
+  }
+  __device__ __forceinline__ uint32_t entry(const Args& a, uint32_t j) const {
+    return CAMERA ? first + j : (a.q.active[a.bounce & 1] + size_t(s) * a.q.region)[j];
+  }
+  __device__ __forceinline__ bool start(const Args& a, const Frame& f, const Seg& sg, uint32_t p, Walk& w, Stack& st) {
+    float4* const ray_o = a.q.ray_o;
+    float4* const ray_d = a.q.ray_d;
+    float4 o4, d4;
+    if (CAMERA) {
+      if (f.cam.max_depth == 0) {  // ray_color with no bounce is black
+        a.q.radiance[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+        return false;
+      }
+      uint32_t x, y, sample;
+      path_coords(f, sg, p, &x, &y, &sample);
+      Rng rng{stream_seed(pixel_seed(f.cam.seed, x, y), sample, 0)};
+      f3 o, d;
+      float time;
+      camera_ray(f.cam, x, y, sample, rng, &o, &d, &time);
+      o4 = make_float4(o.x, o.y, o.z, time);
+      d4 = make_float4(d.x, d.y, d.z, 0.f);
+      ray_o[p] = o4;
+      ray_d[p] = d4;
+    } else {
+      o4 = ray_o[p];
+      d4 = ray_d[p];
+    }
+    walk_begin(f.scene, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), o4.w, CAMERA ? kNoSelf : ray_self(d4.w), w, st);
+    return true;
+  }
+  __device__ __forceinline__ void retire(const Args& a, bool fin, uint32_t p, const Walk& w, const WalkScene& sc) {
+    const bool hit = fin && w.best != kNoPrim, miss = fin && w.best == kNoPrim;
+    const unsigned long long mh = __ballot(hit), mm = __ballot(miss);
+    if (hit) {
+      a.q.hits[p] = make_float2(w.closest, __uint_as_float(w.best));
+      // a camera path has no radiance yet; its throughput and MIS weight are 1, which shade
+      // assumes at bounce 0 without reading them
+      if (CAMERA) a.q.radiance[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+      const uint32_t meta = __float_as_uint(sc.prims[w.best].p0[3]);
+      ring_hit[(hit0 + nhit + rank_below(mh)) % kRing] = (p - first) | (category_of(meta) << 29);
+    }
+    if (miss) ring_miss[(miss0 + nmiss + rank_below(mm)) % kRing] = p;
+    nhit += uint32_t(__popcll(mh));
+    nmiss += uint32_t(__popcll(mm));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if (nhit >= 64u) flush_hits(a, 64u);
+    if (nmiss >= 64u) flush_misses(a, 64u);
+  }
+};
+
+template <bool COUNT, bool MULTI, bool CAMERA, bool WIDE>
 // Traversal kernels run at 8 waves per SIMD (at most 64 VGPRs, a few spilled
 // values): more waves hide more of the dependent node-fetch latency. On one
 // MI355X this took the 720p terrain's extend from 14.6 to 13.8 ms per frame
 // and the Cornell frame from 5.0 to 4.8 ms; a 5-wave target for the shade
 // kernels was slower.
-__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_extend(Frame f0, Batch bt, Queues q, uint32_t bounce) {
+__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_extend(Args) {
   extern __shared__ uint2 smem[];
-  Stack st = make_stack(q, smem);
+  Stack st = make_stack(kernel_args().q, smem);
   for (uint32_t s = blockIdx.x % slice_step(); s < kSlices; s += slice_step()) {
-  const uint32_t count = q.ctr[ctr_at(bounce, S_QCOUNT, s)];
-  if (count == 0) continue;
-  const uint32_t first = CAMERA ? q.ctr[ctr_at(0, S_BASE, s)] : 0;
-  const uint32_t* __restrict__ active = q.active[bounce & 1] + size_t(s) * q.region;
-  const uint32_t per_lane = items_per_lane(count);
-  for (;;) {
-    uint32_t base = wave_fetch(q.ctr + ctr_at(bounce, S_EXT_WORK, s), per_lane);
-    if (base >= count) break;
+    const Args& a = kernel_args();
+    uint32_t* const ctr = a.q.ctr;
+    const uint32_t count = ctr[ctr_at(a.bounce, S_QCOUNT, s)];
+    if (count == 0) continue;
+    uint32_t* const ring = reinterpret_cast<uint32_t*>(smem + blockDim.x * a.q.stack_cap) + (threadIdx.x >> 6) * kRingWords;
+    ExtendPolicy<MULTI, CAMERA> pol{s, ctr[ctr_at(0, S_BASE, s)], ring, ring + kRing};
     uint32_t nodes = 0, prims = 0;
-    uint32_t ids[kChunk], cats[kChunk];
-#pragma unroll
-    for (uint32_t k = 0; k < kChunk; ++k) {
-      uint32_t j = base + k * 64u + lane_id();
-      cats[k] = kNumCategories;
-      ids[k] = 0;
-      const bool valid = k < per_lane && j < count;
-      const uint32_t p = !valid ? 0u : CAMERA ? first + j : active[j];
-      ids[k] = p;
-      with_frame<MULTI>(f0, bt, valid, p, [&](const Frame& f, const Seg& sg) {
-        float4 o4, d4;
-        if (CAMERA) {
-          if (f.cam.max_depth == 0) {  // ray_color with no bounce is black
-            q.radiance[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-            return;
-          }
-          uint32_t x, y, sample;
-          path_coords(f, sg, p, &x, &y, &sample);
-          Rng rng{stream_seed(pixel_seed(f.cam.seed, x, y), sample, 0)};
-          f3 o, d;
-          float time;
-          camera_ray(f.cam, x, y, sample, rng, &o, &d, &time);
-          o4 = make_float4(o.x, o.y, o.z, time);
-          d4 = make_float4(d.x, d.y, d.z, 0.f);
-          q.ray_o[p] = o4;  // stored before the trace: holding the ray across it costs registers
-          q.ray_d[p] = d4;
-        } else {
-          o4 = q.ray_o[p];
-          d4 = q.ray_d[p];
-        }
-        float t;
-        uint32_t prim, meta = 0;
-        Stats s{0, 0, 0, 0, 0, 0};
-        bool hit = trace<false, COUNT>(f.scene, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), o4.w, SHADOW_ACNE, INF,
-                                       CAMERA ? kNoSelf : ray_self(d4.w), st, &t, &prim, nullptr, &s, &meta);
-        if (hit) {
-          q.hits[p] = make_float2(t, __uint_as_float(prim));
-          // a camera path has no radiance yet; its throughput and MIS weight are 1, which shade
-          // assumes at bounce 0 without reading them
-          if (CAMERA) q.radiance[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-          cats[k] = category_of(meta);
-        } else {
-          // a miss ends the path here (camera.rs:1747-1750): background or environment, times the
-          // MIS weight; shading it in place saves a queue and a launch per bounce
-          const float4 t4 = CAMERA ? make_float4(1.f, 1.f, 1.f, 1.f) : q.thr[p];
-          const f3 d = mk(d4.x, d4.y, d4.z);
-          float mw = t4.w;
-          const f3 rad = f.env.kind != 0 ? env_radiance_weighted(f.env, d, &mw) : background(f.cam, d);
-          const f3 miss = rad * mw;
-          const float4 L = CAMERA ? make_float4(0.f, 0.f, 0.f, 0.f) : q.radiance[p];
-          q.radiance[p] = make_float4(L.x + t4.x * miss.x, L.y + t4.y * miss.y, L.z + t4.z * miss.z, 0.f);
-        }
-        if (COUNT) { nodes += node_fetches(s, f.scene.width); prims += s.candidates; }
-      });
-    }
-#pragma unroll
-    for (uint32_t c = CAT_EMIT; c < kNumCategories; ++c) {  // misses were shaded above
-      uint32_t bits = 0;
-#pragma unroll
-      for (uint32_t k = 0; k < kChunk; ++k) bits |= uint32_t(cats[k] == c) << k;
-      wave_append_chunk(q.ctr + ctr_at(bounce, S_CAT_COUNT + c, s), q.cat[c] + size_t(s) * q.region, bits, ids);
-    }
+    walk_queue<MULTI, WIDE, false, COUNT>(st, ctr + ctr_at(a.bounce, S_EXT_WORK, s), count, CAMERA ? 0u : a.q.refill_at,
+                                          pol, nodes, prims);
+    const Args& e = kernel_args();
+    while (pol.nhit) pol.flush_hits(e, min(pol.nhit, 64u));
+    while (pol.nmiss) pol.flush_misses(e, min(pol.nmiss, 64u));
     if (COUNT) {
-      wave_count(count_slot(q, bounce, 0), nodes);
-      wave_count(count_slot(q, bounce, 1), prims);
+      wave_count(count_slot(e.q, e.bounce, 0), nodes);
+      wave_count(count_slot(e.q, e.bounce, 1), prims);
     }
-  }
   }
 }
 
@@ -583,70 +737,64 @@ __global__ void k_shade(Frame f0, Batch bt, Queues q, uint32_t bounce) {
   shade_category<CAT_SPECULAR, MULTI, CAMERA>(f0, bt, q, bounce);
 }
 
-// Shadow rays of one kind. Light targets: closest hit, then the emission of
-// whatever was hit (camera.rs:2248-2261). Environment: any hit occludes
-// (camera.rs:2284-2293; "is some hit" equals "is some closest hit").
-template <bool COUNT, bool MULTI>
-__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_connect(Frame f0, Batch bt, Queues q, uint32_t bounce,
-                                                                   uint32_t kind) {
-  extern __shared__ uint2 smem[];
-  Stack st = make_stack(q, smem);
-  const float4* __restrict__ sd = q.s_d[kind];
-  const float4* __restrict__ sw = q.s_w[kind];
-  for (uint32_t s = blockIdx.x % slice_step(); s < kSlices; s += slice_step()) {
-  const uint32_t count = q.ctr[ctr_at(bounce, kind == 0 ? S_SL_COUNT : S_SE_COUNT, s)];
-  if (count == 0) continue;
-  uint32_t* cursor = q.ctr + ctr_at(bounce, kind == 0 ? S_SL_WORK : S_SE_WORK, s);
-  const uint32_t* __restrict__ list = q.shadow[kind] + size_t(s) * q.region;
-  const uint32_t per_lane = items_per_lane(count);
-  for (;;) {
-    uint32_t base = wave_fetch(cursor, per_lane);
-    if (base >= count) break;
-    uint32_t nodes = 0, prims = 0;
-    for (uint32_t k = 0; k < per_lane; ++k) {
-      const uint32_t j = base + k * 64u + lane_id();
-      const bool valid = j < count;
-      const uint32_t p = valid ? list[j] : 0u;
-      with_frame<MULTI>(f0, bt, valid, p, [&](const Frame& f, const Seg&) {
-      Stats s{0, 0, 0, 0, 0, 0};
-      const float4 o4 = q.ray_o[p], d4 = sd[p];  // the origin is the shading vertex
-      f3 o = mk(o4.x, o4.y, o4.z), d = mk(d4.x, d4.y, d4.z);
-      const uint32_t self = __float_as_uint(d4.w);  // the shading vertex's primitive
-      float t;
-      uint32_t prim;
-      f3 add = mk(0.f, 0.f, 0.f);
-      bool contributes = false;
-      if (kind == 0) {
-        if (trace<false, COUNT>(f.scene, o, d, o4.w, SHADOW_ACNE, INF, self, st, &t, &prim, nullptr, &s)) {
-          f3 pt = o + t * d;
-          uint32_t mid, pk;
-          f3 outward = prim_outward_normal(f.scene.prims, prim, pt, o4.w, &mid, &pk);
-          const GMat& m = f.scene.mats[mid];
-          if (m.kind == GM_DIFFUSE_LIGHT && dot(d, outward) < 0.f) {
-            f3 em = ld3(m.color);
-            if (finite3(em)) { add = em; contributes = true; }
-          }
+// Shadow rays of one kind. Light targets (KIND 0): closest hit, then the
+// emission of whatever was hit (camera.rs:2248-2261). Environment (KIND 1): any
+// hit occludes (camera.rs:2284-2293; "is some hit" equals "is some closest hit").
+template <bool MULTI, int KIND>
+struct ConnectPolicy {
+  uint32_t s;
+  __device__ __forceinline__ uint32_t entry(const Args& a, uint32_t j) const {
+    return (a.q.shadow[KIND] + size_t(s) * a.q.region)[j];
+  }
+  __device__ __forceinline__ bool start(const Args& a, const Frame& f, const Seg&, uint32_t p, Walk& w, Stack& st) {
+    const float4 o4 = a.q.ray_o[p], d4 = a.q.s_d[KIND][p];  // origin: the shading vertex; d4.w: its primitive
+    walk_begin(f.scene, mk(o4.x, o4.y, o4.z), mk(d4.x, d4.y, d4.z), o4.w, __float_as_uint(d4.w), w, st);
+    return true;
+  }
+  __device__ __forceinline__ void retire(const Args& a, bool fin, uint32_t p, const Walk& w, const WalkScene& sc) {
+    f3 add = mk(1.f, 1.f, 1.f);
+    bool contributes = fin && w.best == kNoPrim;
+    if (KIND == 0) {
+      contributes = false;
+      with_frame<MULTI>(a.f, a.bt, fin && w.best != kNoPrim, p, [&](const Frame& f, const Seg&) {
+        const f3 pt = w.o + w.closest * w.d;
+        uint32_t mid, pk;
+        const f3 outward = prim_outward_normal(sc.prims, w.best, pt, w.time, &mid, &pk);
+        const GMat& m = f.scene.mats[mid];
+        if (m.kind == GM_DIFFUSE_LIGHT && dot(w.d, outward) < 0.f) {
+          const f3 em = ld3(m.color);
+          if (finite3(em)) { add = em; contributes = true; }
         }
-      } else {
-        if (!trace<true, COUNT>(f.scene, o, d, o4.w, SHADOW_ACNE, INF, self, st, &t, &prim, nullptr, &s)) {
-          add = mk(1.f, 1.f, 1.f);
-          contributes = true;
-        }
-      }
-      if (contributes) {  // the weight is read only for a ray that lands
-        const float4 w4 = sw[p];
-        add = mul(mk(w4.x, w4.y, w4.z), add);
-        float4 L = q.radiance[p];
-        q.radiance[p] = make_float4(L.x + add.x, L.y + add.y, L.z + add.z, 0.f);
-      }
-      if (COUNT) { nodes += node_fetches(s, f.scene.width); prims += s.candidates; }
       });
     }
-    if (COUNT) {
-      wave_count(count_slot(q, bounce, 2), nodes);
-      wave_count(count_slot(q, bounce, 3), prims);
+    if (contributes) {  // the weight is read only for a ray that lands
+      const float4 w4 = a.q.s_w[KIND][p];
+      add = mul(mk(w4.x, w4.y, w4.z), add);
+      float4* const radiance = a.q.radiance;
+      const float4 L = radiance[p];
+      radiance[p] = make_float4(L.x + add.x, L.y + add.y, L.z + add.z, 0.f);
     }
   }
+};
+
+template <bool COUNT, bool MULTI, bool WIDE, int KIND>
+__global__ __attribute__((amdgpu_waves_per_eu(8))) void k_connect(Args) {
+  extern __shared__ uint2 smem[];
+  Stack st = make_stack(kernel_args().q, smem);
+  for (uint32_t s = blockIdx.x % slice_step(); s < kSlices; s += slice_step()) {
+    const Args& a = kernel_args();
+    uint32_t* const ctr = a.q.ctr;
+    const uint32_t count = ctr[ctr_at(a.bounce, KIND == 0 ? S_SL_COUNT : S_SE_COUNT, s)];
+    if (count == 0) continue;
+    ConnectPolicy<MULTI, KIND> pol{s};
+    uint32_t nodes = 0, prims = 0;
+    walk_queue<MULTI, WIDE, KIND == 1, COUNT>(st, ctr + ctr_at(a.bounce, KIND == 0 ? S_SL_WORK : S_SE_WORK, s), count,
+                                              a.q.refill_at, pol, nodes, prims);
+    if (COUNT) {
+      const Args& e = kernel_args();
+      wave_count(count_slot(e.q, e.bounce, 2), nodes);
+      wave_count(count_slot(e.q, e.bounce, 3), prims);
+    }
   }
 }
 
@@ -820,7 +968,7 @@ __global__ void k_aov(Frame f, Queues q, float* albedo, float* normal) {
       uint32_t prim;
       camera_ray(f.cam, x, y, s, rng, &o, &d, &time);
       PrimHit ph{0.f, 0.f, 0.f};
-      if (trace<false, false>(f.scene, o, d, time, SHADOW_ACNE, INF, kNoSelf, st, &t, &prim, &ph, nullptr)) {
+      if (trace<false>(f.scene, o, d, time, SHADOW_ACNE, INF, kNoSelf, st, &t, &prim, &ph, nullptr)) {
         refine_hit(f.scene.prims, prim, o, d, time, SHADOW_ACNE, &ph);
         t = ph.t;
         f3 p = o + t * d;
@@ -858,7 +1006,7 @@ __global__ void k_intersect(Frame f, Queues q, const float4* __restrict__ rays, 
     uint32_t prim = 0;
     PrimHit ph{0.f, 0.f, 0.f};
     Stats s{0, 0, 0, 0, 0, 0};
-    bool hit = trace<false, STATS>(f.scene, o, d, o4.w, tmin, d4.w, kNoSelf, st, &t, &prim, &ph, &s);
+    bool hit = trace<STATS>(f.scene, o, d, o4.w, tmin, d4.w, kNoSelf, st, &t, &prim, &ph, &s);
     if (hit) {
       refine_hit(f.scene.prims, prim, o, d, o4.w, tmin, &ph);  // the chosen primitive's t, u, v in FP64
       t = ph.t;
@@ -911,11 +1059,15 @@ __global__ void k_zero_words(unsigned long long* p, uint32_t n) {
 uint32_t occupancy_blocks(int kernel, uint32_t block, size_t lds) {
   int nb = 0;
   hipError_t e = hipSuccess;
-  if (kernel == 0) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_extend<false, false, false>, int(block), lds);
+  if (kernel == 0) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_extend<false, false, false, false>, int(block), lds);
   else if (kernel == 1) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_shade<false, false>, int(block), 0);
-  else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_connect<false, false>, int(block), lds);
+  else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_connect<false, false, false, 1>, int(block), lds);
   if (e != hipSuccess || nb <= 0) return 1;
   return uint32_t(nb);
+}
+
+size_t extend_lds_bytes(uint32_t block, uint32_t cap) {
+  return stack_lds_bytes(block, cap) + size_t(block / 64) * kRingWords * sizeof(uint32_t);
 }
 
 // The one place that decides which bounce's extend generates camera rays;
@@ -931,23 +1083,33 @@ void reset_counters(const Launch& l, const Queues& q, uint32_t depth, uint32_t t
 void zero_acc(const Launch& l, double4* acc, size_t n) {
   hipLaunchKernelGGL(k_zero, dim3(l.grid), dim3(l.block), 0, l.stream, acc, n);
 }
-void extend(const Launch& l, const Work& w, const Queues& q, uint32_t bounce, bool count) {
-  const size_t lds = stack_lds_bytes(l.block, q.stack_cap);
-#define GT_EXTEND(C, M, K) \
-  hipLaunchKernelGGL((k_extend<C, M, K>), dim3(l.grid), dim3(l.block), lds, l.stream, w.f, w.bt, q, bounce)
-#define GT_EXTEND_CM(K)                                                  \
-  if (w.multi) {                                                         \
-    if (count) GT_EXTEND(true, true, K); else GT_EXTEND(false, true, K); \
-  } else {                                                               \
-    if (count) GT_EXTEND(true, false, K); else GT_EXTEND(false, false, K); \
-  }
-  if (camera_bounce(bounce)) {
-    GT_EXTEND_CM(true)
+template <bool COUNT, bool MULTI, bool CAMERA, bool WIDE>
+static void launch_extend(const Launch& l, const Work& w, const Queues& q, uint32_t bounce) {
+  const size_t lds = extend_lds_bytes(l.block, q.stack_cap);
+  static const hipError_t attr =  // once per instantiation: blocks of 1024 threads take more than 64 KiB
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_extend<COUNT, MULTI, CAMERA, WIDE>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
+  (void)attr;
+  hipLaunchKernelGGL((k_extend<COUNT, MULTI, CAMERA, WIDE>), dim3(l.grid), dim3(l.block), lds, l.stream,
+                     Args{w.f, w.bt, q, bounce});
+}
+template <bool COUNT, bool MULTI>
+static void extend_cm(const Launch& l, const Work& w, const Queues& q, uint32_t bounce) {
+  const bool cam = camera_bounce(bounce);
+  if (w.wide) {
+    if (cam) launch_extend<COUNT, MULTI, true, true>(l, w, q, bounce);
+    else launch_extend<COUNT, MULTI, false, true>(l, w, q, bounce);
   } else {
-    GT_EXTEND_CM(false)
+    if (cam) launch_extend<COUNT, MULTI, true, false>(l, w, q, bounce);
+    else launch_extend<COUNT, MULTI, false, false>(l, w, q, bounce);
   }
-#undef GT_EXTEND_CM
-#undef GT_EXTEND
+}
+void extend(const Launch& l, const Work& w, const Queues& q, uint32_t bounce, bool count) {
+  if (w.multi) {
+    if (count) extend_cm<true, true>(l, w, q, bounce); else extend_cm<false, true>(l, w, q, bounce);
+  } else {
+    if (count) extend_cm<true, false>(l, w, q, bounce); else extend_cm<false, false>(l, w, q, bounce);
+  }
 }
 void shade(const Launch& l, const Work& w, const Queues& q, uint32_t bounce) {
 #define GT_SHADE(M, K) \
@@ -959,16 +1121,24 @@ void shade(const Launch& l, const Work& w, const Queues& q, uint32_t bounce) {
   }
 #undef GT_SHADE
 }
-void connect(const Launch& l, const Work& w, const Queues& q, uint32_t bounce, uint32_t kind, bool count) {
+template <bool COUNT, bool MULTI>
+static void connect_cm(const Launch& l, const Work& w, const Queues& q, uint32_t bounce, uint32_t kind) {
   const size_t lds = stack_lds_bytes(l.block, q.stack_cap);
-#define GT_CONNECT(C, M) \
-  hipLaunchKernelGGL((k_connect<C, M>), dim3(l.grid), dim3(l.block), lds, l.stream, w.f, w.bt, q, bounce, kind)
-  if (w.multi) {
-    if (count) GT_CONNECT(true, true); else GT_CONNECT(false, true);
+#define GT_CONNECT(W, K) \
+  hipLaunchKernelGGL((k_connect<COUNT, MULTI, W, K>), dim3(l.grid), dim3(l.block), lds, l.stream, Args{w.f, w.bt, q, bounce})
+  if (w.wide) {
+    if (kind == 0) GT_CONNECT(true, 0); else GT_CONNECT(true, 1);
   } else {
-    if (count) GT_CONNECT(true, false); else GT_CONNECT(false, false);
+    if (kind == 0) GT_CONNECT(false, 0); else GT_CONNECT(false, 1);
   }
 #undef GT_CONNECT
+}
+void connect(const Launch& l, const Work& w, const Queues& q, uint32_t bounce, uint32_t kind, bool count) {
+  if (w.multi) {
+    if (count) connect_cm<true, true>(l, w, q, bounce, kind); else connect_cm<false, true>(l, w, q, bounce, kind);
+  } else {
+    if (count) connect_cm<true, false>(l, w, q, bounce, kind); else connect_cm<false, false>(l, w, q, bounce, kind);
+  }
 }
 // One thread per pixel (not the persistent grid): each pixel's loop over its
 // samples is a chain of dependent loads, so more threads hide more of it.

@@ -1,0 +1,80 @@
+"""The traversal kernels' waves, which take new rays as others finish: every
+result is the ray's own, whatever the queue length, launch shape, stack split
+and node width. Bit-exact comparisons: the paths are the same, so the images are.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from gartus_amd import abi, api, scenes  # noqa: E402
+
+
+def _scene(kind):
+    if kind == "few":      # below the node count at which waves refill
+        data, lights, cam = scenes.cornell()
+        cam.pop("grid")
+        targets = api.SamplingTargetList()
+        for _, q, _ in lights:
+            targets.add_quad(q[0:3], q[3:6], q[6:9])
+        return api.RayScene(data), targets, None, dict(cam, spp=2)
+    if kind == "lights":   # many primitives of mixed kinds, light connections
+        data, lights, cam = scenes.batch_scene(1003)
+        targets = api.SamplingTargetList()
+        for _, q, _ in lights:
+            targets.add_quad(q[0:3], q[3:6], q[6:9])
+        return api.RayScene(data), targets, None, dict(cam, spp=2)
+    if kind == "deep":     # a tree deeper than the LDS part of the stack
+        data, cam = scenes.terrain(grid=64, n_spheres=50)
+        return api.RayScene(data), None, None, dict(cam, spp=2)
+    data, env, cam = scenes.ggx_environment(n_random=150, env_size=(64, 32))
+    return api.RayScene(data), None, api.EnvironmentLight.from_rgb32f(env), dict(cam, spp=2)
+
+
+def _camera(spec, w, h):
+    c = api.RayCamera.__new__(api.RayCamera)
+    c.raw = scenes.camera_record(dict(spec, width=w, aspect=w / (h + 0.5)))
+    if "nee" in spec:
+        c.raw.direct_lighting_mode = abi.GT_LIGHTING_NEE
+    return c
+
+
+@pytest.mark.parametrize("kind", ["few", "lights", "deep", "environment"])
+def test_results_do_not_depend_on_queue_length_or_launch_shape(kind):
+    scene, lights, env, spec = _scene(kind)
+    ctx = scene.context
+    cam = _camera(spec, 97, 61)
+    full = api.PathTracer(cam)._render(scene, cam, lights, env).pixels.reshape(-1, 3)
+    assert np.isfinite(full).all() and full.std() > 0
+    # queues of 1, 2 n, ... paths: below, at and above a wave and a claim
+    order = np.random.default_rng(5).permutation(len(full))
+    for n in (1, 31, 32, 33, 63, 64, 65, 129, 1023):
+        px = order[:n]
+        got = api.render_pixels(scene, cam, px, lights, env, double=False)
+        np.testing.assert_array_equal(got, full[px], err_msg=f"{kind}, {n} pixels")
+    old = ctx.tuning
+    try:
+        for shape in (dict(block_size=64), dict(block_size=192, stack_lds=4), dict(block_size=1024),
+                      dict(blocks_per_cu=1), dict(max_paths=1000)):
+            ctx.set_tuning(**shape)
+            got = api.PathTracer(cam)._render(scene, cam, lights, env).pixels.reshape(-1, 3)
+            np.testing.assert_array_equal(got, full, err_msg=f"{kind}, {shape}")
+            ctx.set_tuning(block_size=old.block_size, stack_lds=old.stack_lds, blocks_per_cu=old.blocks_per_cu,
+                           max_paths=old.max_paths)
+    finally:
+        ctx.set_tuning(block_size=old.block_size, stack_lds=old.stack_lds, blocks_per_cu=old.blocks_per_cu,
+                       max_paths=old.max_paths)
+
+
+def test_wide_nodes_render_the_binary_trees_image():
+    """Node width changes the visiting order only; ties aside the hits are the same."""
+    scene, lights, env, spec = _scene("deep")
+    ctx = scene.context
+    cam = _camera(spec, 97, 61)
+    full = api.PathTracer(cam)._render(scene, cam, lights, env).pixels.reshape(-1, 3)
+    try:
+        ctx.set_tuning(bvh_width=4, stack_lds=4)
+        wide = api.PathTracer(cam)._render(scene, cam, lights, env).pixels.reshape(-1, 3)
+    finally:
+        ctx.set_tuning(bvh_width=2, stack_lds=0)
+    assert (wide == full).all(axis=1).mean() > 0.999
