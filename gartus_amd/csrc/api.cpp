@@ -134,6 +134,7 @@ struct gt_env {
   bool uniform = true;
   DevBuf<float4> tex;  // (r, g, b, solid-angle pdf) per texel
   DevBuf<uint2> alias;  // (keep threshold, alias texel) per texel
+  DevBuf<float> row_cos;  // cos of the rows' edges
 };
 
 namespace {
@@ -432,6 +433,13 @@ int make_camera(const gt_camera* c, GCamera* g) {
   return GT_OK;
 }
 
+// Div31 of d in [1, 2^31]: exact quotients of every n < 2^31.
+gtd::Div31 make_div31(uint32_t d) {
+  uint32_t l = 0;
+  while ((uint64_t(1) << l) < d) ++l;
+  return {d, uint32_t((uint64_t(1) << (31 + l)) / d + 1), 31 + l};
+}
+
 gtd::DScene device_scene(const gt_scene* s, uint32_t width) {
   gtd::DScene d;
   d.nodes2 = s->nodes2.p;
@@ -547,6 +555,11 @@ int make_frame(gt_context* ctx, const gt_scene* scene, const gt_camera* camera, 
     f->env.w = env->w; f->env.h = env->h;
     f->env.uniform = env->uniform ? 1u : 0u;
     f->env.tex = env->tex.p; f->env.alias = env->alias.p;
+    f->env.row_cos = env->row_cos.p;
+    if (env->kind == 2) {
+      f->env.row = make_div31(env->w);
+      f->env.inv_w = 1.0f / float(env->w);
+    }
   }
   f->nee = camera->direct_lighting_mode == GT_LIGHTING_NEE ? 1u : 0u;
   f->has_lights = lights ? 1u : 0u;
@@ -554,6 +567,7 @@ int make_frame(gt_context* ctx, const gt_scene* scene, const gt_camera* camera, 
   f->npix = f->cam.width * f->cam.height;
   f->nact = f->npix;
   f->pixmap = nullptr;
+  f->by_width = make_div31(std::max(f->cam.width, 1u));
   return GT_OK;
 }
 
@@ -676,6 +690,7 @@ int run_jobs(gt_context* ctx, std::vector<FrameJob>& jobs, bool multi, int out_i
   uint64_t off = 0;
   for (FrameJob& j : jobs) {
     j.f.acc = ctx->acc.p + off;
+    j.f.by_nact = make_div31(std::max(j.f.nact, 1u));
     off += j.f.npix;
   }
   size_t seg_total = 0;
@@ -1505,7 +1520,9 @@ int gt_env_create_rgb32f(gt_context* ctx, const float* rgb, uint32_t w, uint32_t
     for (size_t i = 0; i < n; ++i) alias[i] = make_uint2(thr[i], idx[i]);
   }
   GT_HIP(hipSetDevice(ctx->device));
-  GT_HIP(e->tex.ensure(n)); GT_HIP(e->alias.ensure(n));
+  GT_HIP(e->tex.ensure(n)); GT_HIP(e->alias.ensure(n)); GT_HIP(e->row_cos.ensure(size_t(h) + 1));
+  gtk::env_rows(ctx->stream, e->row_cos.p, h);
+  GT_HIP(hipGetLastError());
   GT_HIP(hipMemcpy(e->tex.p, tex.data(), n * sizeof(float4), hipMemcpyHostToDevice));
   GT_HIP(hipMemcpy(e->alias.p, alias.data(), n * sizeof(uint2), hipMemcpyHostToDevice));
   *out = e.release();

@@ -85,6 +85,7 @@ struct Frame {
   // only the pixels still sampling); nact = npix and no map otherwise.
   const uint32_t* pixmap;
   uint32_t nact;
+  gtd::Div31 by_nact, by_width;  // of a path's index in its segment, and of a pixel's
 };
 
 // Per-pixel state of adaptive sampling (render_world_pixel_adaptive,
@@ -162,6 +163,8 @@ void aov(const Launch& l, const Frame& f, const Queues& q, float* albedo, float*
 // (6 words) and the largest stack depth (1 word), added to what it holds.
 void intersect(const Launch& l, const Frame& f, const Queues& q, const float4* rays, size_t n, float tmin,
                float4* hits, unsigned long long* stats);
+// Fills row_cos[0..h] (DEnv::row_cos).
+void env_rows(hipStream_t stream, float* row_cos, uint32_t h);
 // Sets n 64-bit words to zero with a kernel (no memset node under capture).
 void zero_words(hipStream_t stream, unsigned long long* p, uint32_t n);
 

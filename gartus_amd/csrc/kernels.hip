@@ -91,11 +91,10 @@ __device__ __forceinline__ Stack make_stack(const Queues& q, uint2* smem) {
 __device__ __forceinline__ void path_coords(const Frame& f, const Seg& sg, uint32_t path, uint32_t* x, uint32_t* y,
                                             uint32_t* sample) {
   const uint32_t local = path - sg.path0;
-  const uint32_t idx = local % f.nact;
+  uint32_t idx;
+  *sample = sg.sample0 + div31(local, f.by_nact, &idx);
   const uint32_t pixel = f.pixmap ? f.pixmap[idx] : idx;
-  *sample = sg.sample0 + local / f.nact;
-  *x = pixel % f.cam.width;
-  *y = pixel / f.cam.width;
+  *y = div31(pixel, f.by_width, x);
 }
 
 // Index of the segment holding `key` in a table sorted by `field`
@@ -163,7 +162,7 @@ __device__ __forceinline__ bool rr_survives(uint32_t bounce, int32_t min_depth, 
 __device__ __forceinline__ float scattering_pdf(const GMat& m, f3 d_in, f3 n, f3 ns, f3 dir) {
   if (m.kind == GM_LAMBERTIAN) {
     float c = dot(ns, normalized(dir));
-    return c <= 0.f ? 0.f : c / PI;
+    return c <= 0.f ? 0.f : div_rn(c, PI, INV_PI);
   }
   if (m.kind == GM_GGX) {
     f3 outgoing = -normalized(d_in);
@@ -174,7 +173,7 @@ __device__ __forceinline__ float scattering_pdf(const GMat& m, f3 d_in, f3 n, f3
   if (m.kind == GM_ISOTROPIC) return 1.0f / (4.0f * PI);
   if (m.kind == GM_HENYEY_GREENSTEIN) {  // HenyeyGreensteinPdf::new(ray_in.direction, g).value
     const f3 w = normalized(d_in);
-    const float l = sqrtf(len2(dir));
+    const float l = sqrt_rn(len2(dir));
     if (len2(w) <= EPS || l <= EPS) return 0.f;
     return hg_phase(dot(dir, w) / l, m.param);
   }
@@ -645,7 +644,7 @@ __device__ __forceinline__ uint32_t shade_specular(const Frame& f, const Queues&
     float ratio = front ? 1.0f / m.param : m.param;
     f3 unit = normalized(it.d);
     float ct = fminf(dot(-unit, n), 1.0f);
-    float stt = sqrtf(1.0f - ct * ct);
+    float stt = sqrt_rn(1.0f - ct * ct);
     bool cannot = ratio * stt > 1.0f;
     float r0 = (1.0f - ratio) / (1.0f + ratio);
     r0 = r0 * r0;
@@ -924,6 +923,11 @@ __global__ void k_adapt_finalize(const double4* mean, const uint32_t* map, uint3
   }
 }
 
+__global__ void k_env_rows(float* row_cos, uint32_t h) {
+  const uint32_t y = blockIdx.x * blockDim.x + threadIdx.x;
+  if (y <= h) row_cos[y] = env_row_cos(y, h);
+}
+
 // Clears accumulators with a kernel (no memset node, so the sequence can be
 // captured in a graph and replayed).
 __global__ void k_zero(double4* acc, size_t n) {
@@ -1189,6 +1193,9 @@ void intersect(const Launch& l, const Frame& f, const Queues& q, const float4* r
   else
     hipLaunchKernelGGL(k_intersect<false>, dim3(l.grid), dim3(l.block), stack_lds_bytes(l.block, q.stack_cap),
                        l.stream, f, q, rays, n, tmin, hits, stats);
+}
+void env_rows(hipStream_t stream, float* row_cos, uint32_t h) {
+  hipLaunchKernelGGL(k_env_rows, dim3(h / 256 + 1), dim3(256), 0, stream, row_cos, h);
 }
 void zero_words(hipStream_t stream, unsigned long long* p, uint32_t n) {
   hipLaunchKernelGGL(k_zero_words, dim3((n + 255) / 256), dim3(256), 0, stream, p, n);
