@@ -15,12 +15,14 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 namespace gdn {
 
 namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
@@ -294,22 +296,10 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ x, co
   }
 }
 
-// ---- convolution, forward: persistent blocks, halos copied straight to LDS --
-// The same tiles and MFMA steps as k_conv, for layers of up to 48 output
-// channels (one group). A block keeps the layer's weights in LDS for its
-// whole life and walks a run of tiles. A tile's input channels run in chunks
-// of 16*GMAX that never straddle the two parts of a decoder concatenation;
-// a (tile, chunk) pair is one stage. The halo of stage s + 1 is copied from
-// global memory into the second of two LDS buffers by buffer loads that
-// write LDS directly (no registers), while the waves run the MFMA steps of
-// stage s; border pixels are read at an offset past the buffer's range and
-// land as zeros. The halo has no padding: piece q (16 bytes) of pixel p sits
-// at slot p * 2G + (q ^ swz<G>(p)), and the weights likewise by row. Blocks are dealt
-// round-robin to the 8 XCDs; each XCD's blocks walk one contiguous eighth of
-// the tiles, so tiles that share halo rows are read through the same L2.
 typedef __attribute__((address_space(3))) void lds_void;
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kOutOfRange = 0x80000000u;  // a buffer offset past every tensor this kernel reads
+constexpr uint32_t kOutOfRange = 0x80000000u;  // a buffer offset past every tensor
 constexpr int kWaitVm0 = 0x0F70;    // s_waitcnt vmcnt(0)
 constexpr int kWaitLgkm0 = 0xC07F;  // s_waitcnt lgkmcnt(0)
 
@@ -322,62 +312,6 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_s_barrier();
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
-
-// The halo buffers hold a chunk of up to 16*GMAX channels in whole 64-slot
-// copies. The output tile is staged in the buffer it was computed from, in
-// passes of at most 32 channels (bf16; 16 channels fp32 for the network
-// output): 256 pixels x the pass's channels, rows padded by 16 bytes when the
-// padded pass still fits.
-template <int NT, bool OUT_F32>
-constexpr int pipe_pass_channels() {
-  return OUT_F32 ? 16 : std::min(NT * 16, 32);
-}
-template <int NT, bool OUT_F32>
-constexpr int pipe_passes() {
-  return (NT * 16 + pipe_pass_channels<NT, OUT_F32>() - 1) / pipe_pass_channels<NT, OUT_F32>();
-}
-template <int NT, bool OUT_F32>
-constexpr int pipe_raw_row_bytes() {  // one pass
-  return pipe_pass_channels<NT, OUT_F32>() * (OUT_F32 ? 4 : 2);
-}
-template <int NT, bool OUT_F32, int GMAX>
-constexpr int pipe_buf_slots() {
-  return std::max((kHR * kHC * 2 * GMAX + 63) / 64 * 64, 256 * pipe_raw_row_bytes<NT, OUT_F32>() / 16);
-}
-template <int NT, bool OUT_F32, int GMAX>
-constexpr int pipe_row_bytes() {
-  constexpr int raw = pipe_raw_row_bytes<NT, OUT_F32>();
-  return 256 * (raw + 16) <= pipe_buf_slots<NT, OUT_F32, GMAX>() * 16 ? raw + 16 : raw;
-}
-template <int NT, bool OUT_F32>
-constexpr int pipe_row_pieces() {  // 16-byte pieces of one output pixel
-  return OUT_F32 ? NT * 4 : NT * 2;
-}
-constexpr int pipe_pool_per_thread(int nt) { return (2 * 32 * nt * 2 + 255) / 256; }
-
-// Chunks of a layer's input: channels [0, ca) of the half-resolution part
-// first, then [ca, cin) of the full-resolution part, each in runs of 16*GMAX
-// channels and a last run of 16 when GMAX is 2 and the part has an odd
-// number of 16-channel groups.
-struct PipeChunk {
-  int c0, g;
-  bool half_res;
-};
-template <int GMAX>
-__device__ __forceinline__ int pipe_nchunks(int cin, int ca) {
-  constexpr int CS = 16 * GMAX;
-  return (ca + CS - 1) / CS + (cin - ca + CS - 1) / CS;
-}
-template <int GMAX>
-__device__ __forceinline__ PipeChunk pipe_chunk(int k, int cin, int ca) {
-  constexpr int CS = 16 * GMAX;
-  const int na = (ca + CS - 1) / CS;
-  if (k < na) return {CS * k, std::min(GMAX, (ca - CS * k) / 16), true};
-  const int c0 = ca + CS * (k - na);
-  return {c0, std::min(GMAX, (cin - c0) / 16), false};
-}
-
-typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 // A raw buffer resource over [base, base + bytes): reads past the end return
 // zeros.
@@ -408,306 +342,373 @@ __device__ __forceinline__ void lds_copy16(const uint4* dst, i32x4 src, uint32_t
 #pragma clang diagnostic pop
 }
 
-// Issues the copies of one chunk's halo into buf: wave w copies slots
-// [64 i, 64 i + 64) for i = w, w + 4, ... Channel c of the source (src_c
-// channels per pixel) is the chunk's first.
-template <int G>
-__device__ __forceinline__ void pipe_copy_halo(uint4* buf, i32x4 src, int src_c, int c,
-                                               bool half_res, int n, int h0, int w0, int H, int W, int wave,
-                                               int lane) {
-  constexpr int QP = 2 * G, SL = kHR * kHC * QP, NI = (SL + 63) / 64;
-  const int Hs = half_res ? H / 2 : H, Ws = half_res ? W / 2 : W;
-#pragma unroll
-  for (int i0 = 0; i0 < NI; i0 += 4) {
-    const int i = i0 + wave;
-    if (i < NI) {
-      const int s = i * 64 + lane, px = s / QP;
-      const int q = (s % QP) ^ swz<G>(px);
-      const int hh = h0 - 1 + px / kHC, ww = w0 - 1 + px % kHC;
-      uint32_t off = kOutOfRange;
-      if (s < SL && hh >= 0 && hh < H && ww >= 0 && ww < W) {
-        const int sh = half_res ? hh >> 1 : hh, sw = half_res ? ww >> 1 : ww;
-        off = uint32_t((((size_t(n) * Hs + sh) * Ws + sw) * src_c + c + 8 * q) * 2);
-      }
-      lds_copy16(buf + i * 64, src, off);
-    }
-  }
-}
+// ---- convolution by rows: weights in registers, pixels straight from global memory --
+// Forward and data gradient for the layer shapes of launch_rows. A wave owns a
+// strip of 16 pixel columns and NT * 16 output channels and walks down the rows
+// of a segment. The roles of the MFMA operands are swapped against k_conv:
+// A holds weights (M = output channels), B pixels (N = 16 columns), so that
+//   - the layer's weights stay in registers for the wave's whole life;
+//   - a pixel fragment, read once, serves the three output rows it touches;
+//   - a lane ends with 4 NT consecutive channels of one pixel (fragment j's row
+//     4 g + r is channel 4 NT g + 4 j + r), which it stores as they are: no
+//     staging in LDS, no barrier anywhere.
+// A fragment is one 16-byte buffer load per lane (16 pixels); columns and rows
+// outside the image are read past the buffer's range and arrive as zeros. Every
+// load and store is such a buffer access, so a row's body has no branch and the
+// waits for the loads in flight are exact; the loads run PF rows ahead.
+//
+// Sums are made in a fixed order, the same as k_conv's and as the persistent kernel's that this one replaced: by
+// groups of input channels, tap by tap within one. A group of 32 channels takes one K = 32 MFMA step per tap. A group
+// of 16 pairs taps (0,1), (2,3), (4,5), (6,7), (8,-) in the two halves of K. A part's odd 16 channels are such a group;
+// with PAIRS all are. Its fragments, of row i, are the column taps F = (-1 | 0), G = (+1 | -1) and H = (0 | +1), and
+// output row r takes F(r-1), G(r-1) with the upper half of G(r), H(r), F(r+1), G(r+1) with zeros. Two groups side by
+// side are loaded as one of 32 channels, three contiguous loads a row, and their fragments made by exchanging register
+// halves: loading them as they are takes six loads of 32-byte pieces, and 32->32 took 72 us for 60 at 1920x1080.
+//
+// What bounds it, on one MI355X at 1920x1080: the full-resolution layers of 16 and 32 channels move 3.7 to 4.9 TB/s,
+// near what a copy reaches; the wide ones run one wave per SIMD, whose instruction stream (MFMA steps, exchanges,
+// packing) then bounds them. With the pixels through LDS, as in k_conv, 64 pixels x 32 channels x 32 outputs cost 6 LDS
+// reads per 8 MFMA steps, more than the LDS delivers. Without the empty asm statements below, weights are copied from
+// accumulation registers on each use and row offsets become branches around the loads: 48+32->32 took 152 us, not 117.
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 
-// The MFMA steps of one chunk (G 16-channel groups) from the swizzled halo
-// and the chunk's weights from slot wb of wts (rows tap * NT*16 + co, 2G
-// pieces each, swizzled the same way by row). Both arrays are indexed from
-// their bases in one step.
-template <int NT, int G, bool MIRROR>
-__device__ __forceinline__ void pipe_chunk_mfma(const uint4* halo, const uint4* wts, int wb, int lane, int wave,
-                                                v4f (&acc)[4][NT]) {
-  constexpr int QP = 2 * G;
-  const int half = (lane >> 4) & 1, col = lane & 15;
-#pragma unroll
-  for (int i = 0; i < (9 * G + 1) / 2; ++i) {
-    const int sub = 2 * i + (lane >> 5);
-    const bool valid = sub < 9 * G;
-    const int tap = valid ? sub / G : 0;
-    const int q = (sub % G) * 2 + half;
-    const int dy = MIRROR ? 1 - tap / 3 : tap / 3 - 1, dx = MIRROR ? 1 - tap % 3 : tap % 3 - 1;
-    uint4 b[NT];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) {
-      const int r = tap * NT * 16 + j * 16 + col;
-      b[j] = valid ? wts[wb + r * QP + (q ^ swz<G>(r))] : make_uint4(0, 0, 0, 0);
-    }
-    const int p0 = (wave + 1 + dy) * kHC + col + 1 + dx;
-#pragma unroll
-    for (int f = 0; f < 4; ++f) {
-      const int p = p0 + 16 * f;
-      const uint4 a = valid ? halo[p * QP + (q ^ swz<G>(p))] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < NT; ++j) acc[f][j] = mfma32(a, b[j], acc[f][j]);
-    }
-  }
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {  // round to nearest even
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v2f{lo, hi}, v2bf));
 }
+__device__ __forceinline__ float relu_of(float v) { return __builtin_amdgcn_fmed3f(v, 0.f, __builtin_huge_valf()); }
 
-// A finished tile's output, read back from its LDS staging into registers:
-// this wave's row (pieces lane, lane + 64, ...) and this thread's pieces of
-// the 2x2 max pool. The stores are issued one step later, right after the
-// next halo copy, so that the wait for that copy does not also wait for them.
-template <int NT, bool OUT_F32>
-struct PipeOut {
-  u32x4 row[pipe_row_pieces<NT, OUT_F32>()];  // vector types, not uint4: they stay in registers
-  u32x4 pool[pipe_pool_per_thread(NT)];
-  u32x4 mrow[OUT_F32 ? 1 : pipe_row_pieces<NT, OUT_F32>()];  // the output mask of the row pieces
-  int tile = -1;
+constexpr int kRowsBytes = 0x40000000;  // a segment's rows of any tensor take less
+struct RowsJob {  // a launch's tensors and shape
+  const uint16_t* x;    // the full-resolution part, CB channels
+  const uint16_t* xa;   // the half-resolution part, CA channels (CA > 0)
+  const uint16_t* wgt;  // [cout][9][CA + CB]
+  const float* bias;
+  void* y;              // bf16 [n][h][w][cout]; ROWS_F32 fp32; ROWS_RADIANCE fp32 [n][rh][rw][3]
+  uint16_t* pooled;     // ROWS_POOL: 2x2 max pool of y
+  const uint16_t* omask;  // ROWS_GRAD_MASK
+  int rh, rw;
+  int cout, co_first;
+  int N, H, W;
+  int nseg, nstrip, seg_rows, groups;  // row segments and strips of an image; output groups of NT * 16 channels
+};
+// Forward (bias, ReLU), the same with the pooled copy, data gradient (taps mirrored), the same masked by the ReLU
+// of the tensor it belongs to, network output z, network output as radiance expm1(max(z, 0)) of channels 0..2.
+enum RowsMode { ROWS_FWD, ROWS_POOL, ROWS_GRAD, ROWS_GRAD_MASK, ROWS_F32, ROWS_RADIANCE };
+
+// The units of an input of CA + CB channels, in order: 32 channels each, then a part's odd 16.
+template <int CA, int CB, bool PAIRS>
+struct RowsPlan {
+  static constexpr int WA = CA / 32, OA = CA / 16 % 2, WB = CB / 32, OB = CB / 16 % 2;
+  static constexpr int NC = WA + OA + WB + OB;
+  static constexpr int WIDE = PAIRS ? 10 : 9, ODD = 5;  // MFMA steps of a unit, per output row and fragment
+  static constexpr int STEPS = WIDE * (WA + WB) + ODD * (OA + OB);
+  static constexpr bool in_a(int c) { return c < WA + OA; }
+  static constexpr int local(int c) { return in_a(c) ? c : c - WA - OA; }  // within its part
+  static constexpr bool odd(int c) { return local(c) >= (in_a(c) ? WA : WB); }
+  static constexpr int first(int c) { return 32 * local(c); }  // first channel within its part
+  static constexpr int steps(int c) { return odd(c) ? ODD : WIDE; }
+  static constexpr int step0(int c) {  // the unit's first MFMA step
+    int s = 0;
+    for (int k = 0; k < c; ++k) s += steps(k);
+    return s;
+  }
 };
 
-// Bias and ReLU of the accumulators, staged through buf (bf16, or fp32 for the
-// network output) pass by pass and read back into out; clears acc for the
-// next tile. With rad (the network output only) lane l keeps instead the
-// radiance expm1(max(z, 0)) of channels 0..2 of its pixel, the wave's row's
-// pixel l.
-template <int NT, bool OUT_F32, int GMAX>
-__device__ __forceinline__ void pipe_finish(uint4* buf, v4f (&acc)[4][NT], const float (&bj)[NT], int relu,
-                                            bool pooled, bool rad, PipeOut<NT, OUT_F32>& out, int t, int tid,
-                                            int lane, int wave, const uint16_t* omask, int cout, int co0, int H,
-                                            int W, int nrt, int nct) {
-  if (!OUT_F32 && omask) {
-    // the output mask of this lane's row pieces, loaded now: the next step's wait for its halo
-    // copy (issued before these loads) covers them, so the stores wait for nothing more
-    constexpr int GP = pipe_row_pieces<NT, OUT_F32>();
-    const int ct = t % nct, rt = (t / nct) % nrt, n = t / (nct * nrt);
-    const int row = rt * kTR + wave, w0 = ct * kTC;
-#pragma unroll
-    for (int k = 0; k < GP; ++k) {
-      const int i = lane + 64 * k, p = i / GP, g = i % GP;
-      out.mrow[k] = u32x4{0u, 0u, 0u, 0u};
-      if (row < H && w0 + p < W)
-        out.mrow[k] = *reinterpret_cast<const u32x4*>(omask + ((size_t(n) * H + row) * W + w0 + p) * cout + co0 + 8 * g);
-    }
-  }
-  constexpr int RB = pipe_row_bytes<NT, OUT_F32, GMAX>(), GP = pipe_row_pieces<NT, OUT_F32>();
-  constexpr int PC = pipe_pass_channels<NT, OUT_F32>(), PJ = PC / 16;  // channels, fragments per pass
-  constexpr int CP = OUT_F32 ? 4 : 8;                                  // channels per 16-byte piece
-  char* st = reinterpret_cast<char*>(buf);
-#pragma unroll
-  for (int pass = 0; pass < pipe_passes<NT, OUT_F32>(); ++pass) {
-    lds_barrier();  // every wave is done with buf: the halo, or the previous pass
-#pragma unroll
-    for (int jj = 0; jj < PJ; ++jj) {
-      const int j = pass * PJ + jj;
-      if (j >= NT) break;
-#pragma unroll
-      for (int f = 0; f < 4; ++f)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float v = acc[f][j][r] + bj[j];
-          if (relu) v = fmaxf(v, 0.f);
-          const int px = wave * 64 + f * 16 + (lane >> 4) * 4 + r, c = jj * 16 + (lane & 15);
-          if (OUT_F32) *reinterpret_cast<float*>(st + px * RB + 4 * c) = v;
-          else *reinterpret_cast<uint16_t*>(st + px * RB + 2 * c) = f2bf(v);
-          acc[f][j][r] = 0.f;
-        }
-    }
-    lds_barrier();
-    const int g0 = pass * PC / CP, g1 = std::min(GP, (pass + 1) * PC / CP);  // this pass's pieces
-    if (OUT_F32 && rad) {
-      const float* z = reinterpret_cast<const float*>(st + (wave * 64 + lane) * RB);
-      out.row[0] = u32x4{__float_as_uint(expm1f(fmaxf(z[0], 0.f))), __float_as_uint(expm1f(fmaxf(z[1], 0.f))),
-                         __float_as_uint(expm1f(fmaxf(z[2], 0.f))), 0u};
-    } else {
-#pragma unroll
-      for (int k = 0; k < GP; ++k) {
-        const int i = lane + 64 * k, p = i / GP, g = i % GP;
-        if (g >= g0 && g < g1) out.row[k] = *reinterpret_cast<const u32x4*>(st + (wave * 64 + p) * RB + 16 * (g - g0));
-      }
-    }
-    if (!OUT_F32 && pooled) {  // the staged values are already bf16: the max of them is the pooled value
-      constexpr int G8 = NT * 2;
-#pragma unroll
-      for (int k = 0; k < pipe_pool_per_thread(NT); ++k) {
-        const int i = tid + 256 * k;
-        const int g = i % G8, pc = (i / G8) % 32, pr = i / (G8 * 32);
-        if (i >= 2 * 32 * G8 || g < g0 || g >= g1) continue;
-        const char* a = st + ((2 * pr) * 64 + 2 * pc) * RB + 16 * (g - g0);
-        const u32x4 v[4] = {*reinterpret_cast<const u32x4*>(a), *reinterpret_cast<const u32x4*>(a + RB),
-                            *reinterpret_cast<const u32x4*>(a + 64 * RB),
-                            *reinterpret_cast<const u32x4*>(a + 65 * RB)};
-        u32x4 o;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t w[4] = {v[0][e], v[1][e], v[2][e], v[3][e]};
-          float lo = bf2f(uint16_t(w[0])), hi = bf2f(uint16_t(w[0] >> 16));
-#pragma unroll
-          for (int m = 1; m < 4; ++m) {
-            lo = fmaxf(lo, bf2f(uint16_t(w[m])));
-            hi = fmaxf(hi, bf2f(uint16_t(w[m] >> 16)));
-          }
-          o[e] = uint32_t(f2bf(lo)) | (uint32_t(f2bf(hi)) << 16);
-        }
-        out.pool[k] = o;
-      }
-    }
-  }
-  out.tile = t;
-}
+template <int CA, int CB, bool PAIRS, int NT, RowsMode MODE, int WAVES, int PF, int LDSA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES))) void k_conv_rows(RowsJob q) {
+  using P = RowsPlan<CA, CB, PAIRS>;
+  constexpr int CIN = CA + CB, NC = P::NC, BW = 3 + PF;  // BW: rows of a fragment ring
+  constexpr bool F32 = MODE == ROWS_F32 || MODE == ROWS_RADIANCE;
+  constexpr bool MIRROR = MODE == ROWS_GRAD || MODE == ROWS_GRAD_MASK;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, g = lane >> 4;
+  // blocks are dealt round-robin to the 8 XCDs; an XCD's blocks share one contiguous eighth of the
+  // tiles, four of a block at a time (one a wave), and a block keeps its output channels
+  const int ntile = q.N * q.nseg * q.nstrip, xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+  const int t0 = int(int64_t(ntile) * xcd / 8) + wave, t1 = int(int64_t(ntile) * (xcd + 1) / 8);
+  const int per = (gridDim.x >> 3) / q.groups;  // blocks of an XCD with the same channels
+  const int co0 = q.co_first + slot % q.groups * (NT * 16);
+  const int cl = co0 + 4 * NT * g;              // this lane's first output channel
 
-// The global stores of a finished tile held in out. With rad: radiance
-// [n][rh][rw][3] of the pixels inside rh x rw (the caller's image in the
-// padded tensor), instead of y.
-template <int NT, bool OUT_F32>
-__device__ __forceinline__ void pipe_store(PipeOut<NT, OUT_F32>& out, void* y, uint16_t* pooled, float* rad, int rh,
-                                           int rw, const uint16_t* omask, int cout, int co0, int H, int W, int nrt,
-                                           int nct, int tid, int lane, int wave) {
-  constexpr int GP = pipe_row_pieces<NT, OUT_F32>();
-  const int t = out.tile;
-  out.tile = -1;
-  const int ct = t % nct, rt = (t / nct) % nrt, n = t / (nct * nrt);
-  const int h0 = rt * kTR, w0 = ct * kTC;
-  const int row = h0 + wave;
-  if (OUT_F32 && rad) {
-    if (row < rh && w0 + lane < rw) {
-      float* o = rad + ((size_t(n) * rh + row) * rw + w0 + lane) * 3;
-      o[0] = __uint_as_float(out.row[0][0]);
-      o[1] = __uint_as_float(out.row[0][1]);
-      o[2] = __uint_as_float(out.row[0][2]);
-    }
-  } else if (row < H) {
-    const size_t pix0 = (size_t(n) * H + row) * W;
+  // the weights, step by step: this lane's piece of each fragment; the last LDSA steps' in LDS
+  constexpr int AREG = P::STEPS - LDSA;
+  u32x4 A[AREG][NT];
+  __shared__ u32x4 Al[LDSA ? LDSA : 1][NT][64];
 #pragma unroll
-    for (int k = 0; k < GP; ++k) {
-      const int i = lane + 64 * k, p = i / GP, g = i % GP;
-      if (w0 + p >= W) continue;
-      if (OUT_F32) {
-        *reinterpret_cast<u32x4*>(static_cast<float*>(y) + (pix0 + w0 + p) * cout + co0 + 4 * g) = out.row[k];
+  for (int c = 0; c < NC; ++c) {
+    const bool pair = P::odd(c) || PAIRS;
+    const int c0 = (P::in_a(c) ? 0 : CA) + P::first(c);
+#pragma unroll
+    for (int i = 0; i < P::steps(c); ++i) {
+      const int tap = pair ? 2 * (i % 5) + (g >> 1) : i, ch = c0 + (pair ? 16 * (i / 5) + 8 * (g & 1) : 8 * g);
+      const bool live = tap < 9;
+      const int t = live ? (MIRROR ? 8 - tap : tap) : 0;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int co = co0 + 4 * NT * (col >> 2) + 4 * j + (col & 3);
+        u32x4 v = *reinterpret_cast<const u32x4*>(q.wgt + (size_t(co) * 9 + t) * CIN + ch);
+        if (!live) v = u32x4{0u, 0u, 0u, 0u};
+        const int step = P::step0(c) + i;
+        if (step < AREG) A[step < AREG ? step : 0][j] = v;
+        else if (wave == 0) Al[step - AREG][j][lane] = v;
+      }
+    }
+  }
+  // matrix operands only: kept in accumulation registers, which leaves the others to the pixels
+#pragma unroll
+  for (int i = 0; i < AREG; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) asm volatile("" : "+a"(A[i][j]));
+  v4f bj[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) bj[j] = MIRROR ? v4f{0.f, 0.f, 0.f, 0.f} : *reinterpret_cast<const v4f*>(q.bias + cl + 4 * j);
+
+  if (LDSA) __syncthreads();
+
+  for (int tile = t0 + slot / q.groups * 4; tile < t1; tile += per * 4) {
+    const int strip = tile % q.nstrip, sg = (tile / q.nstrip) % q.nseg, n = tile / (q.nstrip * q.nseg);
+    const int r0 = sg * q.seg_rows, r1 = min(r0 + q.seg_rows, q.H), w = strip * 16 + col;
+    const int i0 = max(r0 - 1, 0), i1 = min(r1 + 1, q.H);  // input rows read
+    // buffers over the rows this job reads and writes, so that offsets stay small for tensors of any size
+    constexpr int kRaw = 0x00020000;
+    const int pb = q.W * CB * 2, Wa = q.W >> 1, pa = Wa * CA * 2, a0 = i0 >> 1;
+    const auto rb = __builtin_amdgcn_make_buffer_rsrc((void*)(q.x + (size_t(n) * q.H + i0) * q.W * CB), 0, (i1 - i0) * pb, kRaw);
+    const auto ra = __builtin_amdgcn_make_buffer_rsrc((void*)(CA ? q.xa + (size_t(n) * (q.H >> 1) + a0) * Wa * CA : q.x), 0,
+                                                      CA ? (((i1 + 1) >> 1) - a0) * pa : 0, kRaw);
+    const int py = MODE == ROWS_RADIANCE ? q.rw * 12 : q.W * q.cout * (F32 ? 4 : 2);  // output bytes per row
+    const int yrows = MODE == ROWS_RADIANCE ? max(min(r1, q.rh) - r0, 0) : r1 - r0;
+    const size_t ybase = MODE == ROWS_RADIANCE ? (size_t(n) * q.rh + r0) * q.rw * 12 : (size_t(n) * q.H + r0) * py;
+    const auto ry = __builtin_amdgcn_make_buffer_rsrc(static_cast<char*>(q.y) + ybase, 0, yrows * py, kRaw);
+    const int yoff = MODE == ROWS_RADIANCE ? (g == 0 && w < q.rw ? w * 12 : int(kOutOfRange))
+                                           : (w < q.W ? (w * q.cout + cl) * (F32 ? 4 : 2) : int(kOutOfRange));
+    const auto rm = __builtin_amdgcn_make_buffer_rsrc(
+        MODE == ROWS_GRAD_MASK ? (void*)(reinterpret_cast<const char*>(q.omask) + ybase) : q.y, 0,
+        MODE == ROWS_GRAD_MASK ? yrows * py : 0, kRaw);
+    const int pp = (q.W >> 1) * q.cout * 2;
+    const auto rp = __builtin_amdgcn_make_buffer_rsrc(
+        MODE == ROWS_POOL ? (void*)(reinterpret_cast<char*>(q.pooled) + (size_t(n) * (q.H >> 1) + (r0 >> 1)) * pp) : q.y, 0,
+        MODE == ROWS_POOL ? ((r1 - r0) >> 1) * pp : 0, kRaw);
+    const int poff = (col & 1) == 0 && w < q.W ? ((w >> 1) * q.cout + cl) * 2 : int(kOutOfRange);
+    // this lane's byte offset in a row of a part at column tap dx, or past every buffer
+    auto offset = [&](bool a, int dx, int ch) {
+      const int ww = w + dx;
+      return dx < 2 && ww >= 0 && ww < q.W ? ((a ? ww >> 1 : ww) * (a ? CA : CB) + ch) * 2 : int(kOutOfRange);
+    };
+    const int hi = g >> 1, c8 = 8 * g, p8 = 8 * (g & 1);
+    int of[2][2][3];  // [part][odd unit][fragment]
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) of[a][0][k] = offset(a == 0, k - 1, c8);
+      of[a][1][0] = offset(a == 0, hi ? 0 : -1, p8);
+      of[a][1][1] = offset(a == 0, hi ? -1 : 1, p8);
+      of[a][1][2] = offset(a == 0, hi ? 1 : 0, p8);
+    }
+    // a row outside the image; less than kOutOfRange, so that the two can be added
+    constexpr int kRowOut = kRowsBytes;
+    const int rows = r1 - r0;
+    u32x4 B[NC][3][BW];  // fragment ring: row r0 - 1 + m in slot m % BW
+    u32x2 M[NT][BW];     // ROWS_GRAD_MASK: the output mask of row r0 + m in slot m % BW
+    // Byte offsets of input row r0 - 1 + m in both parts, past the buffer outside the image. Read back as
+    // uniform values, they stay selects, where a branch around each load would serialise the loads.
+    struct RowAt { int a, b; };
+    auto row_of = [&](int m) {
+      const int i = r0 - 1 + m;
+      const bool in = uint32_t(i - i0) < uint32_t(i1 - i0);
+      const int a = __builtin_amdgcn_readfirstlane(((i >> 1) - a0) * pa), b = __builtin_amdgcn_readfirstlane((i - i0) * pb);
+      return RowAt{__builtin_amdgcn_readfirstlane(in ? a : kRowOut), __builtin_amdgcn_readfirstlane(in ? b : kRowOut)};
+    };
+    // Fragment k of the units of 32 channels or of the odd ones, row r0 - 1 + m.
+    auto load = [&](auto S, bool odd, int k, RowAt r) {
+      constexpr int slot_ = decltype(S)::value;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        if (P::odd(c) != odd) continue;
+        const bool a = P::in_a(c);
+        B[c][k][slot_] = __builtin_amdgcn_raw_buffer_load_b128(a ? ra : rb, of[a ? 0 : 1][odd][k] + (a ? r.a : r.b) + 2 * P::first(c), 0, 0);
+      }
+    };
+    auto load_mask = [&](auto S, int m) {
+      constexpr int slot_ = decltype(S)::value;
+      if constexpr (MODE == ROWS_GRAD_MASK) {
+        const int sm = yoff + (m < rows ? m * py : kRowOut);
+#pragma unroll
+        for (int j = 0; j + 1 < NT; j += 2) {
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rm, sm + 8 * j, 0, 0);
+          M[j][slot_] = u32x2{v[0], v[1]};
+          M[j + 1][slot_] = u32x2{v[2], v[3]};
+        }
+        if constexpr (NT & 1) M[NT - 1][slot_] = __builtin_amdgcn_raw_buffer_load_b64(rm, sm + 8 * (NT - 1), 0, 0);
+      }
+    };
+    u32x4 F[NC][2][BW];  // PAIRS: the column taps (-1 | 0) of a unit's two 16-channel halves
+    // The lower and the upper halves of two fragments, side by side: of the same pixels' 32 channels at two taps, the
+    // pair fragments of channels 0..15 and of 16..31.
+    auto halves = [](u32x4 p, u32x4 q2, u32x4& lower, u32x4& upper) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto v = __builtin_amdgcn_permlane32_swap(p[e], q2[e], false, false);
+        lower[e] = v[0];
+        upper[e] = v[1];
+      }
+    };
+    v4f acc[NT];
+    u32x2 prev[NT];  // ROWS_POOL: the row above
+#pragma unroll
+    for (int j = 0; j < NT; ++j) prev[j] = u32x2{0u, 0u};
+    // Output row r0 + m from its sums.
+    auto finish = [&](auto S, int m) {
+      constexpr int slot_ = decltype(S)::value;
+      v4f v[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[j][r] = MIRROR ? acc[j][r] : acc[j][r] + bj[j][r];
+      const int so = yoff + m * py;
+      if constexpr (MODE == ROWS_RADIANCE) {
+        typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+        u32x3 o;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) o[c] = __float_as_uint(expm1f(fmaxf(v[0][c], 0.f)));
+        __builtin_amdgcn_raw_buffer_store_b96(o, ry, so, 0, 0);
+      } else if constexpr (MODE == ROWS_F32) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v[j]), ry, so + 16 * j, 0, 0);
       } else {
-        const size_t off = (pix0 + w0 + p) * cout + co0 + 8 * g;
-        u32x4 v = out.row[k];
-        if (omask) {  // zero where the mask is not positive (the ReLU of the tensor this gradient belongs to)
-          const u32x4 m = out.mrow[k];
+        u32x2 p[NT];
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            v[e] &= (bf2f(uint16_t(m[e])) > 0.f ? 0x0000ffffu : 0u) | (bf2f(uint16_t(m[e] >> 16)) > 0.f ? 0xffff0000u : 0u);
+        for (int j = 0; j < NT; ++j) {
+          if (!MIRROR) p[j] = u32x2{pack_bf16(relu_of(v[j][0]), relu_of(v[j][1])), pack_bf16(relu_of(v[j][2]), relu_of(v[j][3]))};
+          else p[j] = u32x2{pack_bf16(v[j][0], v[j][1]), pack_bf16(v[j][2], v[j][3])};
+          if (MODE == ROWS_GRAD_MASK)  // zero where the mask is not positive
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const uint32_t k = M[j][slot_][e];
+              p[j][e] &= (bf2f(uint16_t(k)) > 0.f ? 0x0000ffffu : 0u) | (__uint_as_float(k & 0xffff0000u) > 0.f ? 0xffff0000u : 0u);
+            }
         }
-        *reinterpret_cast<u32x4*>(static_cast<uint16_t*>(y) + off) = v;
+        auto put = [&](auto rsrc, const u32x2(&d)[NT], int o) {
+#pragma unroll
+          for (int j = 0; j + 1 < NT; j += 2)
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{d[j][0], d[j][1], d[j + 1][0], d[j + 1][1]}, rsrc, o + 8 * j, 0, 0);
+          if constexpr (NT & 1) __builtin_amdgcn_raw_buffer_store_b64(d[NT - 1], rsrc, o + 8 * (NT - 1), 0, 0);
+        };
+        put(ry, p, so);
+        if constexpr (MODE == ROWS_POOL) {  // the stored values are already bf16: the max of them is the pooled value
+          u32x2 d[NT];
+#pragma unroll
+          for (int j = 0; j < NT; ++j) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              float lo = fmaxf(bf2f(uint16_t(prev[j][e])), bf2f(uint16_t(p[j][e])));
+              float up = fmaxf(__uint_as_float(prev[j][e] & 0xffff0000u), __uint_as_float(p[j][e] & 0xffff0000u));
+              lo = fmaxf(lo, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(lo), 0xB1, 0xf, 0xf, true)));
+              up = fmaxf(up, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(up), 0xB1, 0xf, 0xf, true)));
+              d[j][e] = (__float_as_uint(lo) >> 16) | (__float_as_uint(up) & 0xffff0000u);
+            }
+            prev[j] = p[j];
+          }
+          put(rp, d, poff + (m & 1 ? (m >> 1) * pp : kRowOut));  // segments start on even rows
+        }
       }
+    };
+    // Step t makes output row r0 + t and reads what step t + PF needs new.
+    auto row = [&](auto T, int t) {
+      constexpr int k = decltype(T)::value;  // t % BW
+      auto at = [](auto i) { return std::integral_constant<int, decltype(i)::value % BW>{}; };
+#define GT_AT(d) at(std::integral_constant<int, k + (d)>{})
+      const RowAt ahead = row_of(t + 2 + PF);
+#pragma unroll
+      for (int f = 0; f < 3; ++f) load(GT_AT(2 + PF), false, f, ahead);
+      if constexpr (P::OA || P::OB) {
+        load(GT_AT(2 + PF), true, 0, ahead);
+        load(GT_AT(2 + PF), true, 1, ahead);
+        load(GT_AT(1 + PF), true, 2, row_of(t + 1 + PF));
+      }
+      load_mask(GT_AT(PF), t + PF);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        constexpr int up = k, mid = (k + 1) % BW, down = (k + 2) % BW;  // slots of the three rows
+        u32x4 b[10];
+        if (P::odd(c)) {
+          b[0] = B[c][0][up];
+          b[2] = B[c][2][mid];
+          b[3] = B[c][0][down];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            b[1][e] = hi ? B[c][1][mid][e] : B[c][1][up][e];
+            b[4][e] = hi ? 0u : B[c][1][down][e];
+          }
+        } else if (PAIRS) {
+          halves(B[c][0][down], B[c][1][down], F[c][0][down], F[c][1][down]);
+          b[0] = F[c][0][up];
+          b[5] = F[c][1][up];
+          halves(B[c][2][up], B[c][0][mid], b[1], b[6]);
+          halves(B[c][1][mid], B[c][2][mid], b[2], b[7]);
+          b[3] = F[c][0][down];
+          b[8] = F[c][1][down];
+          halves(B[c][2][down], u32x4{0u, 0u, 0u, 0u}, b[4], b[9]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 9; ++i) b[i] = B[c][i % 3][(k + i / 3) % BW];
+        }
+#pragma unroll
+        for (int i = 0; i < P::steps(c); ++i) {
+          const int step = P::step0(c) + i;
+#pragma unroll
+          for (int j = 0; j < NT; ++j)
+            acc[j] = mfma32(__builtin_bit_cast(uint4, step < AREG ? A[step < AREG ? step : 0][j]
+                                                                     : Al[step < AREG ? 0 : step - AREG][j][lane]),
+                               __builtin_bit_cast(uint4, b[i]), acc[j]);
+        }
+      }
+      finish(T, t);
+    };
+    // the rows the first PF steps would have asked for
+    auto warm = [&](auto Mv) {
+      constexpr int m = decltype(Mv)::value;
+      if constexpr (m < 2 + PF) {
+        const RowAt r = row_of(m);
+#pragma unroll
+        for (int f = 0; f < 3; ++f) load(Mv, false, f, r);
+        load(Mv, true, 0, r);
+        load(Mv, true, 1, r);
+        if constexpr (m >= 1 && m < 1 + PF) load(Mv, true, 2, r);
+        if constexpr (m < PF) load_mask(Mv, m);
+      }
+    };
+    warm(std::integral_constant<int, 0>{});
+    warm(std::integral_constant<int, 1>{});
+    warm(std::integral_constant<int, 2>{});
+    warm(std::integral_constant<int, 3>{});
+    warm(std::integral_constant<int, 4>{});
+    if constexpr (PAIRS) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        if (!P::odd(c))
+#pragma unroll
+          for (int m = 0; m < 2; ++m) halves(B[c][0][m], B[c][1][m], F[c][0][m], F[c][1][m]);
     }
+#define GT_ROW(K)                                    \
+  if constexpr (K < BW) {                            \
+    row(std::integral_constant<int, K % BW>{}, t);   \
+    if (++t == rows) break;                          \
   }
-  if (!OUT_F32 && pooled) {
-    constexpr int G8 = NT * 2;
-    const int H2 = H / 2, W2 = W / 2;
-#pragma unroll
-    for (int k = 0; k < pipe_pool_per_thread(NT); ++k) {
-      const int i = tid + 256 * k;
-      if (i >= 2 * 32 * G8) break;
-      const int g = i % G8, pc = (i / G8) % 32, pr = i / (G8 * 32);
-      const int h2 = h0 / 2 + pr, w2 = w0 / 2 + pc;
-      if (h2 < H2 && w2 < W2)
-        *reinterpret_cast<u32x4*>(pooled + ((size_t(n) * H2 + h2) * W2 + w2) * cout + co0 + 8 * g) = out.pool[k];
+    for (int t = 0;;) {
+      GT_ROW(0)
+      GT_ROW(1)
+      GT_ROW(2)
+      GT_ROW(3)
+      GT_ROW(4)
+      GT_ROW(5)
     }
+#undef GT_ROW
+#undef GT_AT
   }
-}
-
-template <int NT, bool OUT_F32, int CIN, int GMAX, bool MIRROR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_conv_pipe(const uint16_t* __restrict__ x,
-                                                   const uint16_t* __restrict__ xa, int ca,
-                                                   const uint16_t* __restrict__ wgt, const float* __restrict__ bias,
-                                                   void* __restrict__ y, uint16_t* __restrict__ pooled, int cout,
-                                                   int co_first, int N, int H, int W, int nrt, int nct, int relu,
-                                                   float* __restrict__ rad, int rh, int rw,
-                                                   const uint16_t* __restrict__ omask) {
-  __shared__ uint4 bufA[pipe_buf_slots<NT, OUT_F32, GMAX>()];
-  __shared__ uint4 bufB[pipe_buf_slots<NT, OUT_F32, GMAX>()];
-  __shared__ uint4 wts4[9 * NT * 16 * CIN / 8];
-  constexpr int cin = CIN;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int co0 = co_first + blockIdx.y * NT * 16;
-  const int cx = cin - ca;
-  const i32x4 rx = buffer_rsrc(x, uint32_t(size_t(N) * H * W * cx * 2));
-  const i32x4 ra = buffer_rsrc(xa ? xa : x, xa ? uint32_t(size_t(N) * (H / 2) * (W / 2) * ca * 2) : 0u);
-
-  // this block's tiles: the XCD's eighth of them, every per-th from slot0
-  const int ntiles = N * nrt * nct;
-  const int xcd = blockIdx.x & 7, per = gridDim.x >> 3, slot0 = blockIdx.x >> 3;
-  const int t_begin = int(int64_t(ntiles) * xcd / 8), t_end = int(int64_t(ntiles) * (xcd + 1) / 8);
-  const int mine = t_end - t_begin > slot0 ? (t_end - t_begin - slot0 + per - 1) / per : 0;
-  const int nch = pipe_nchunks<GMAX>(cin, ca);
-  const int S = mine * nch;
-  if (S == 0) return;  // uniform over the block: no barrier is skipped by part of it
-
-  // the weights, once: piece c/8 of row (tap, co) of the chunk holding channel c
-  const int npc = cin / 8;
-  for (int i = tid; i < 9 * NT * 16 * npc; i += 256) {
-    const int cp = i % npc, rt = i / npc, co = rt / 9, tap = rt % 9, c = 8 * cp;
-    constexpr int CS = 16 * GMAX;
-    const int c0 = c < ca ? c / CS * CS : ca + (c - ca) / CS * CS;
-    const int g = std::min(GMAX, ((c < ca ? ca : cin) - c0) / 16);
-    const int r = tap * NT * 16 + co, q = (c - c0) >> 3;
-    const int sw = g == 2 ? swz<2>(r) : swz<1>(r);
-    wts4[9 * NT * 16 * (c0 / 8) + r * 2 * g + (q ^ sw)] =
-        *reinterpret_cast<const uint4*>(wgt + (size_t(co0 + co) * 9 + tap) * cin + c);
-  }
-  float bj[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) bj[j] = bias ? bias[co0 + j * 16 + (lane & 15)] : 0.f;
-
-  auto copy = [&](uint4* buf, int s) {
-    const int k = s / nch, ch = s - k * nch;
-    const int t = t_begin + slot0 + k * per;
-    const int ct = t % nct, rt = (t / nct) % nrt, n = t / (nct * nrt);
-    const PipeChunk c = pipe_chunk<GMAX>(ch, cin, ca);
-    const i32x4 src = c.half_res ? ra : rx;
-    const int src_c = c.half_res ? ca : cx, c_src = c.half_res ? c.c0 : c.c0 - ca;
-    if (GMAX == 2 && c.g == 2)
-      pipe_copy_halo<2>(buf, src, src_c, c_src, c.half_res, n, rt * kTR, ct * kTC, H, W, wave, lane);
-    else pipe_copy_halo<1>(buf, src, src_c, c_src, c.half_res, n, rt * kTR, ct * kTC, H, W, wave, lane);
-  };
-  v4f acc[4][NT];
-#pragma unroll
-  for (int f = 0; f < 4; ++f)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[f][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  PipeOut<NT, OUT_F32> out;
-  auto step = [&](uint4* cur, uint4* nxt, int s) {
-    __builtin_amdgcn_s_waitcnt(kWaitVm0);  // this wave's copies into cur (and its last stores) are done
-    lds_barrier();  // ... and every wave's; nxt was last read in the previous step
-    if (s + 1 < S) copy(nxt, s + 1);
-    if (out.tile >= 0)
-      pipe_store<NT, OUT_F32>(out, y, pooled, rad, rh, rw, omask, cout, co0, H, W, nrt, nct, tid, lane, wave);
-    const int k = s / nch, ch = s - k * nch;
-    const PipeChunk c = pipe_chunk<GMAX>(ch, cin, ca);
-    const int wb = 9 * NT * 16 * (c.c0 / 8);
-    if (GMAX == 2 && c.g == 2) pipe_chunk_mfma<NT, 2, MIRROR>(cur, wts4, wb, lane, wave, acc);
-    else pipe_chunk_mfma<NT, 1, MIRROR>(cur, wts4, wb, lane, wave, acc);
-    if (ch == nch - 1)
-      pipe_finish<NT, OUT_F32, GMAX>(cur, acc, bj, relu, pooled != nullptr, rad != nullptr, out,
-                                     t_begin + slot0 + k * per, tid, lane, wave, omask, cout, co0, H, W, nrt, nct);
-  };
-  copy(bufA, 0);
-  for (int s = 0; s < S; s += 2) {
-    step(bufA, bufB, s);
-    if (s + 1 < S) step(bufB, bufA, s + 1);
-  }
-  if (out.tile >= 0)
-    pipe_store<NT, OUT_F32>(out, y, pooled, rad, rh, rw, omask, cout, co0, H, W, nrt, nct, tid, lane, wave);
 }
 
 // ---- convolution, weight gradient -----------------------------------------
@@ -820,7 +821,6 @@ constexpr size_t wgrad_tr_lds_bytes() {  // two buffers
   return std::max(size_t(2) * (NCO * wgt_dslots<TC>() + NCI * wgt_xslots<TC>()) * 16, kWRed);
 }
 
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef short v4s __attribute__((ext_vector_type(4)));
 
 // The 8 K values of this lane for a 16 x 32 operand whose K runs over the
@@ -1246,95 +1246,98 @@ int device_cus() {
   return n;
 }
 
-// The persistent forward convolution, for the layer shapes where it is faster
-// than k_conv on one MI355X: the default network's full-resolution layers and
-// level 1's 32 -> 48 and 48 -> 48, tensors addressable by 31-bit buffer
-// offsets. These fit two blocks per CU. False for the others, which take
-// k_conv: the decoder's 64 + 48 -> 48 keeps 97 KB of weights resident, one
-// block fits a CU, and it ran 40 % slower than k_conv.
-template <int NT, bool F32, int CIN, int GMAX, bool MIRROR = false>
-bool launch_pipe_nt(hipStream_t s, const uint16_t* x, const uint16_t* xa, int ca, const uint16_t* w,
-                    const float* bias, void* y, uint16_t* pooled, int cout, Dims d, int relu, float* rad = nullptr,
-                    int rh = 0, int rw = 0, const uint16_t* omask = nullptr, int co_first = 0) {
-  if (size_t(d.n) * d.h * d.w * (CIN - ca) * 2 >= kOutOfRange) return false;
-  if (xa && size_t(d.n) * (d.h / 2) * (d.w / 2) * ca * 2 >= kOutOfRange) return false;
-  static const int per_cu = [] {  // resident blocks per CU
-    int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_conv_pipe<NT, F32, CIN, GMAX, MIRROR>, 256, 0) !=
-            hipSuccess ||
-        n <= 0)
-      n = 1;
-    return n;
-  }();
-  const int nrt = (d.h + kTR - 1) / kTR, nct = (d.w + kTC - 1) / kTC;
-  const int ntiles = d.n * nrt * nct;
-  const int nb = (std::min(ntiles, device_cus() * per_cu) + 7) / 8 * 8;  // a multiple of the 8 XCDs
-  hipLaunchKernelGGL((k_conv_pipe<NT, F32, CIN, GMAX, MIRROR>), dim3(nb, 1), dim3(256), 0, s, x, xa, ca, w, bias, y,
-                     pooled, cout, co_first, d.n, d.h, d.w, nrt, nct, relu, rad, rh, rw, omask);
+// How an instance is built: waves per SIMD (512 registers per lane, shared), rows read ahead (1 to 3), and steps
+// whose weights stay in LDS.
+template <int WAVES_, int PF_, int LDSA_ = 0>
+struct RowsCfg {
+  static constexpr int WAVES = WAVES_, PF = PF_, LDSA = LDSA_;
+};
+
+template <int CA, int CB, bool PAIRS, int NT, RowsMode MODE, class CFG>
+bool launch_rows_nt(hipStream_t s, RowsJob q) {
+  const int waves = device_cus() * 4 * CFG::WAVES;
+  q.nstrip = (q.W + 15) / 16;
+  // rows per segment: the fewest rows in sequence, each segment costing two rows more than it makes
+  int best = 0;
+  int64_t best_cost = INT64_MAX;
+  for (int r : {64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
+    const int64_t jobs = int64_t(q.N) * ((q.H + r - 1) / r) * q.nstrip * q.groups;
+    const int64_t cost = (jobs + waves - 1) / waves * (std::min(r, q.H) + 2);
+    if (cost < best_cost) best = r, best_cost = cost;
+  }
+  const size_t widest = std::max({CA * 2, CB * 2, q.cout * (MODE == ROWS_F32 ? 4 : 2), 12});
+  if (size_t(best + 2) * q.W * widest >= kRowsBytes) return false;
+  q.seg_rows = best;
+  q.nseg = (q.H + best - 1) / best;
+  const int64_t quads = (int64_t(q.N) * q.nseg * q.nstrip + 31) / 32 * q.groups;  // blocks an XCD could use
+  int bpx = int(std::min<int64_t>(quads, std::max(waves / 32, q.groups)));
+  bpx = std::max(bpx / q.groups, 1) * q.groups;
+  hipLaunchKernelGGL((k_conv_rows<CA, CB, PAIRS, NT, MODE, CFG::WAVES, CFG::PF, CFG::LDSA>), dim3(8 * bpx), dim3(256), 0, s, q);
   return true;
 }
 
-// The data gradient (taps mirrored, input already masked) through the same
-// kernel, for the full-resolution shapes that fit one group; omask zeroes the
-// output where the forward tensor it belongs to is not positive.
-bool launch_pipe_dgrad(hipStream_t s, const uint16_t* x, int cin, const uint16_t* w, void* y, int cout, Dims d,
-                       const uint16_t* omask) {
-  // wider outputs (the gradient of the decoder's concatenation, 80 or 112 channels from 32 or 48):
-  // launches of 48 output channels, then one of the rest
-  if (cout > 48 && cout % 16 == 0 && (cin == 32 || cin == 48)) {
-    if (size_t(d.n) * d.h * d.w * std::max(cin, cout) * 2 >= kOutOfRange) return false;
-    for (int c = 0; c < cout;) {
-      const int nt = std::min(3, (cout - c) / 16);
-      if (cin == 32) {
-        if (nt == 3) launch_pipe_nt<3, false, 32, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0,
-                                                            nullptr, 0, 0, omask, c);
-        else if (nt == 2) launch_pipe_nt<2, false, 32, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0,
-                                                                 nullptr, 0, 0, omask, c);
-        else launch_pipe_nt<1, false, 32, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0, nullptr, 0,
-                                                    0, omask, c);
-      } else {
-        if (nt == 3) launch_pipe_nt<3, false, 48, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0,
-                                                            nullptr, 0, 0, omask, c);
-        else if (nt == 2) launch_pipe_nt<2, false, 48, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0,
-                                                                 nullptr, 0, 0, omask, c);
-        else launch_pipe_nt<1, false, 48, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0, nullptr, 0,
-                                                    0, omask, c);
-      }
-      c += 16 * nt;
-    }
-    return true;
-  }
-  switch ((cout / 16) * 1000 + cin) {
-    case 2016:
-      return launch_pipe_nt<2, false, 16, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0, nullptr, 0, 0,
-                                                   omask);
-    case 2032:
-      return launch_pipe_nt<2, false, 32, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0, nullptr, 0, 0,
-                                                   omask);
-    case 2048:
-      return launch_pipe_nt<2, false, 48, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0, nullptr, 0, 0,
-                                                   omask);
-    case 3048:
-      return launch_pipe_nt<3, false, 48, 1, true>(s, x, nullptr, 0, w, nullptr, y, nullptr, cout, d, 0, nullptr, 0, 0,
-                                                   omask);
+template <int CA, int CB, bool PAIRS, int NT, class CFG>
+bool launch_rows_mode(hipStream_t s, const RowsJob& q, RowsMode mode) {
+  switch (mode) {
+    case ROWS_FWD: return launch_rows_nt<CA, CB, PAIRS, NT, ROWS_FWD, CFG>(s, q);
+    case ROWS_POOL: if constexpr (CA == 0) return launch_rows_nt<CA, CB, PAIRS, NT, ROWS_POOL, CFG>(s, q); else return false;
+    case ROWS_GRAD: if constexpr (CA == 0) return launch_rows_nt<CA, CB, false, NT, ROWS_GRAD, CFG>(s, q); else return false;
+    case ROWS_GRAD_MASK: if constexpr (CA == 0) return launch_rows_nt<CA, CB, false, NT, ROWS_GRAD_MASK, CFG>(s, q); else return false;
     default: return false;
   }
 }
 
-template <bool F32>
-bool launch_pipe(hipStream_t s, const uint16_t* x, int cin, const uint16_t* xa, int ca, const uint16_t* w,
-                 const float* bias, void* y, uint16_t* pooled, int cout, Dims d, int relu) {
-  const int key = (cout / 16) * 1000 + cin;
-  if (F32) {
-    if (key == 1032) return launch_pipe_nt<1, true, 32, 1>(s, x, xa, ca, w, bias, y, pooled, cout, d, relu);
-    return false;
+// The output channels in groups of NT fragments; a remainder of 1 to NT - 1 in a launch of its own.
+template <int CA, int CB, bool PAIRS, int NT, class CFG, class CFG1 = CFG, class CFG2 = CFG>
+bool launch_rows_all(hipStream_t s, RowsJob q, RowsMode mode) {
+  const int frags = q.cout / 16, full = frags / NT, rest = frags % NT;
+  q.groups = full;
+  q.co_first = 0;
+  if (full && !launch_rows_mode<CA, CB, PAIRS, NT, CFG>(s, q, mode)) return false;
+  q.groups = 1;
+  q.co_first = full * NT * 16;
+  if constexpr (NT > 1)
+    if (rest == 1) return launch_rows_mode<CA, CB, PAIRS, 1, CFG1>(s, q, mode);
+  if constexpr (NT > 2)
+    if (rest == 2) return launch_rows_mode<CA, CB, PAIRS, 2, CFG2>(s, q, mode);
+  return true;
+}
+
+// The layers that take the row kernel; false for the others, which take k_conv. Measured on one MI355X (us; k_conv or
+// the persistent LDS kernel that stood here before, then this one) on a 1920x1080 frame: 16->32 58 and 54, 32->32 76
+// and 54, 32->48 39 and 29, 48->48 47 and 32, 48->64 32 and 13, 64->64 34 and 22, 64->96 18 and 15, 96->96 22 and 15,
+// 48+32->32 171 and 117, 64+48->48 87 and 53, 96+64->64 62 and 45, the output 52 and 45. Where it lost, the layers stay
+// with k_conv: 128 channels and more in a part (128->128: 14 and 20; a wave's weights fill its registers for a few rows'
+// work). An instance takes as many output channels per wave as its registers hold, which divides the fragment loads by
+// them; the widest keep weights in LDS, and one wave per SIMD beat two that spill.
+//
+// PAIRS follows the layer, in the forward direction, so that a layer's sums are the same whatever kernel makes them:
+// taps pair over 16 channels in the shapes of the default network's full-resolution level and of level 1's 32->48 and
+// 48->48, 32 channels to a tap elsewhere.
+bool launch_rows(hipStream_t s, const RowsJob& q, int ca, int cb, RowsMode mode) {
+  if (mode == ROWS_F32 || mode == ROWS_RADIANCE) {
+    if (ca || cb != 32 || q.cout != 16) return false;
+    RowsJob r = q;
+    r.groups = 1;
+    r.co_first = 0;
+    return mode == ROWS_F32 ? launch_rows_nt<0, 32, true, 1, ROWS_F32, RowsCfg<2, 2>>(s, r)
+                            : launch_rows_nt<0, 32, true, 1, ROWS_RADIANCE, RowsCfg<2, 2>>(s, r);
   }
-  switch (key) {
-    case 2016: return launch_pipe_nt<2, false, 16, 1>(s, x, xa, ca, w, bias, y, pooled, cout, d, relu);
-    case 2032: return launch_pipe_nt<2, false, 32, 1>(s, x, xa, ca, w, bias, y, pooled, cout, d, relu);
-    case 2080: return launch_pipe_nt<2, false, 80, 1>(s, x, xa, ca, w, bias, y, pooled, cout, d, relu);
-    case 3032: return launch_pipe_nt<3, false, 32, 1>(s, x, xa, ca, w, bias, y, pooled, cout, d, relu);
-    case 3048: return launch_pipe_nt<3, false, 48, 1>(s, x, xa, ca, w, bias, y, pooled, cout, d, relu);
+  switch (ca * 1000 + cb) {
+    case 16: return launch_rows_all<0, 16, true, 2, RowsCfg<4, 1>>(s, q, mode);
+    case 32:
+      if (q.cout == 48) return launch_rows_all<0, 32, true, 3, RowsCfg<2, 2>>(s, q, mode);
+      if (q.cout == 32) return launch_rows_all<0, 32, true, 2, RowsCfg<2, 2>>(s, q, mode);
+      return launch_rows_all<0, 32, false, 2, RowsCfg<2, 2>>(s, q, mode);
+    case 48:
+      if (q.cout == 48) return launch_rows_all<0, 48, true, 3, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
+      return launch_rows_all<0, 48, false, 2, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
+    case 64: return launch_rows_all<0, 64, false, 2, RowsCfg<1, 1>, RowsCfg<2, 1>>(s, q, mode);
+    case 96: return launch_rows_all<0, 96, false, 2, RowsCfg<1, 1>>(s, q, mode);
+    case 48032: return q.cout == 32 && launch_rows_all<48, 32, true, 2, RowsCfg<1, 1>, RowsCfg<1, 2>>(s, q, mode);
+    case 64032: return launch_rows_all<64, 32, false, 2, RowsCfg<1, 1>>(s, q, mode);
+    case 64048: return launch_rows_all<64, 48, false, 3, RowsCfg<1, 1, 12>>(s, q, mode);
+    case 96064: return launch_rows_all<96, 64, false, 2, RowsCfg<1, 1, 26>>(s, q, mode);
     default: return false;
   }
 }
@@ -1360,10 +1363,14 @@ template <bool DGRAD, bool F32>
 void launch_conv(hipStream_t s, const uint16_t* x, const uint16_t* mask, int cin, const uint16_t* xa, int ca,
                  const uint16_t* w, const float* bias, void* y, int cout, Dims d, int relu,
                  uint16_t* pooled = nullptr, const uint16_t* omask = nullptr) {
-  if (!DGRAD && launch_pipe<F32>(s, x, cin, xa, ca, w, bias, y, pooled, cout, d, relu)) return;
-  if (DGRAD && !F32 && !mask && !xa && d.n * ((d.h + kTR - 1) / kTR) * ((d.w + kTC - 1) / kTC) >= 1024 &&
-      launch_pipe_dgrad(s, x, cin, w, y, cout, d, omask))
-    return;
+  if (!mask) {
+    RowsJob q{};
+    q.x = x; q.xa = xa; q.wgt = w; q.bias = bias; q.y = y; q.pooled = pooled; q.omask = omask;
+    q.cout = cout; q.N = d.n; q.H = d.h; q.W = d.w;
+    const RowsMode mode = F32 ? ROWS_F32 : DGRAD ? (omask ? ROWS_GRAD_MASK : ROWS_GRAD) : pooled ? ROWS_POOL : ROWS_FWD;
+    const bool like = F32 ? !relu : DGRAD || (relu && !omask);  // a bias with ReLU, or neither, as the modes have them
+    if (like && launch_rows(s, q, xa ? ca : 0, xa ? cin - ca : cin, mode)) return;
+  }
   const int tiles = d.n * ((d.h + kTR - 1) / kTR) * ((d.w + kTC - 1) / kTC);
   const int nt = tiles >= 1024 ? 4 : tiles >= 256 ? 2 : 1;
   const int frags = cout / 16, full = frags / nt, rest = frags % nt;
@@ -1401,7 +1408,9 @@ void conv_fwd(hipStream_t s, const uint16_t* x, int cin, const uint16_t* w, cons
 bool conv_fwd_radiance(hipStream_t s, const uint16_t* x, int cin, const uint16_t* w, const float* bias, float* out,
                        int h, int w_img, Dims d) {
   if (cin != 32) return false;
-  return launch_pipe_nt<1, true, 32, 1>(s, x, nullptr, 0, w, bias, nullptr, nullptr, 16, d, 0, out, h, w_img);
+  RowsJob q{};
+  q.x = x; q.wgt = w; q.bias = bias; q.y = out; q.rh = h; q.rw = w_img; q.cout = 16; q.N = d.n; q.H = d.h; q.W = d.w;
+  return launch_rows(s, q, 0, 32, ROWS_RADIANCE);
 }
 
 void conv_fwd_upcat(hipStream_t s, const uint16_t* a, int ca, const uint16_t* b, int cb, const uint16_t* w,

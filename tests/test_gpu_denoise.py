@@ -103,11 +103,19 @@ def test_forward_and_gradients_match_oracle(gpu_context, levels, channels, n, h,
     _check_forward_and_gradients(gpu_context, levels, channels, n, h, w, loss)
 
 
-# Layers of at least 1,024 tiles of 4 x 64 pixels take the persistent kernel for their data
-# gradients (taps mirrored); the gradient of the decoder's concatenation, 80 channels from 32 or
-# 112 from 48, is split over launches of 48 output channels and the rest. The cases above are too
-# small for it: 128 x 2048 is exactly 1,024 tiles at full resolution. (The oracle takes about 20
-# and 50 s here.)
+# Every channel pair with a row-kernel instance (strips of 16 columns, segments of 2 to 64 rows, output
+# channels in groups of 16 to 48 and a remainder), forward and backward, at widths below, at and beyond a
+# strip, heights of one and several segments, and more strips than a block's four waves.
+@pytest.mark.parametrize("levels,channels,n,h,w", [
+    (2, (32, 48), 1, 2, 2), (2, (32, 48), 3, 17, 15), (2, (32, 64), 1, 6, 130), (2, (48, 64), 1, 66, 18),
+    (2, (48, 64), 1, 64, 260), (2, (64, 96), 2, 10, 34), (2, (96, 128), 1, 5, 33), (2, (96, 128), 1, 131, 16)])
+def test_row_kernel_shapes_match_oracle(gpu_context, levels, channels, n, h, w):
+    _check_forward_and_gradients(gpu_context, levels, channels, n, h, w, abi.GT_DENOISE_LOSS_REL_L2)
+
+
+# The gradient of the decoder's concatenation, 80 channels from 32 or 112 from 48, is split over
+# launches of its output channels; 128 x 2048 at full resolution gives every wave several segments.
+# (The oracle takes about 20 and 50 s here.)
 @pytest.mark.parametrize("channels", [(32, 48), (48, 64)], ids=["cat80", "cat112"])
 def test_persistent_data_gradients_match_oracle(gpu_context, channels):
     _check_forward_and_gradients(gpu_context, 2, channels, 1, 128, 2048, abi.GT_DENOISE_LOSS_REL_L2)
