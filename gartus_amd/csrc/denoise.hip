@@ -1325,6 +1325,8 @@ bool launch_rows(hipStream_t s, const RowsJob& q, int ca, int cb, RowsMode mode)
     case 32:
       if (q.cout == 48) return launch_rows_all<0, 32, true, 3, RowsCfg<2, 2>>(s, q, mode);
       if (q.cout == 32) return launch_rows_all<0, 32, true, 2, RowsCfg<2, 2>>(s, q, mode);
+      // five fragments a wave where they divide: 32->80 in one launch, 66 us at 16x256x256; 61 + 51 in launches of 2 and 1
+      if (q.cout % 80 == 0) return launch_rows_all<0, 32, false, 5, RowsCfg<1, 2>>(s, q, mode);
       return launch_rows_all<0, 32, false, 2, RowsCfg<2, 2>>(s, q, mode);
     case 48:
       if (q.cout == 48) return launch_rows_all<0, 48, true, 3, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
