@@ -456,10 +456,12 @@ gtd::DScene device_scene(const gt_scene* s, uint32_t width) {
   return d;
 }
 
-uint64_t stack_depth(const gt_scene* s, uint32_t width) {
+// Stack entries of a query (trace), and of a render's walk, whose bottom entry ends it (walk_begin).
+uint64_t query_stack_depth(const gt_scene* s, uint32_t width) {
   uint64_t d = width == 4 ? s->packed.depth4 * 3 : s->packed.depth2;  // wide nodes push up to 3 per level
-  return d + 3;  // one entry ends a walk
+  return d + 2;
 }
+uint64_t walk_stack_depth(const gt_scene* s, uint32_t width) { return query_stack_depth(s, width) + 1; }
 
 // LDS traversal-stack entries per lane (gt_tuning.stack_lds); 8 measured
 // fastest on the 1080p GGX/environment frame (occupancy against spills).
@@ -907,7 +909,7 @@ int prepare_job(gt_context* ctx, const gt_scene* cscene, const gt_camera* camera
   j->depth = j->f.cam.max_depth;
   j->conn_l = j->f.nee && lights != nullptr;
   j->conn_e = j->f.nee && env != nullptr;
-  j->stack_need = stack_depth(scene, j->f.scene.width);
+  j->stack_need = walk_stack_depth(scene, j->f.scene.width);
   j->nodes = scene->n_nodes2;
   return GT_OK;
 }
@@ -1329,7 +1331,7 @@ int gt_intersect(gt_context* ctx, const gt_scene* cs, const gt_ray* rays, size_t
   gtk::Frame f;
   std::memset(&f, 0, sizeof f);
   f.scene = device_scene(s, ctx->tuning.bvh_width);
-  if ((rc = ensure_gstack(ctx, stack_depth(s, f.scene.width), stack_cap(ctx))) != GT_OK) return rc;
+  if ((rc = ensure_gstack(ctx, query_stack_depth(s, f.scene.width), stack_cap(ctx))) != GT_OK) return rc;
   gtk::Queues q = queues_of(ctx);
   gtk::Launch L{grid_for(ctx), ctx->tuning.block_size, ctx->stream};
   const size_t chunk = size_t(1) << 22;
@@ -1376,7 +1378,7 @@ int gt_intersect_device_noalloc(gt_context* ctx, const gt_scene* s, const gt_ray
   // Overflow levels of the per-lane stack beyond the LDS entries; the grid
   // shrinks until lanes * levels fits the scratch, down to one block per CU.
   const uint32_t cap = stack_cap(ctx), block = ctx->tuning.block_size;
-  const uint64_t need = stack_depth(s, f.scene.width);
+  const uint64_t need = query_stack_depth(s, f.scene.width);
   const uint64_t levels = need > cap ? need - cap : 1;
   const uint64_t fit_blocks = gtk::kNoAllocStackEntries / (levels * block);
   if (fit_blocks < ctx->cus) {

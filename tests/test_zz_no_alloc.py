@@ -122,3 +122,33 @@ def test_noalloc_intersect_requires_a_built_scene(gpu_context):
         assert b"not built" in lib.gt_last_error()
     finally:
         lib.gt_scene_destroy(h)
+
+
+def test_noalloc_depth_limit_is_the_querys_own(gpu_context):
+    """A tree whose query stack (depth + 2 entries) just fits the scratch is answered, one entry less is
+    refused: the entry that ends a render's walk is not part of a query."""
+    data = scenes.terrain(grid=96, n_spheres=200, seed=5)[0].as_float32_exact()
+    rs = api.RayScene(data).with_bvh()
+    h = rs._compile()
+    ctx = rs.context
+    need = int(rs.info().bvh_depth) + 2
+    cus = 256  # one MI355X
+    old = ctx.tuning
+    # scratch levels at this block size + LDS entries = need
+    block, cap = next((b, need - (1 << 21) // (cus * b)) for b in range(1024, 0, -64)
+                      if 4 < need - (1 << 21) // (cus * b) <= min(32, 8192 // b))
+    rays = _rays(np.random.default_rng(3), 10_000, (-52, -1, -52), (52, 9, 52))
+    say(f"noalloc intersect: {need} stack entries, block {block}, {cap} in LDS")
+    buf = DeviceBuffers(ctx, len(rays))
+    try:
+        ctx.set_tuning(block_size=block, stack_lds=cap)
+        hits, stats = _noalloc_intersect(ctx, h, rays, buf)
+        ref_hits, ref_stats = _host_intersect(ctx, h, rays)
+        np.testing.assert_array_equal(hits.view(np.uint32), ref_hits.view(np.uint32))
+        np.testing.assert_array_equal(stats, ref_stats)
+        ctx.set_tuning(stack_lds=cap - 1)
+        rc = ctx.lib.gt_intersect_device_noalloc(ctx.handle, h, buf.rays, len(rays), C.c_float(0.001), buf.hits, None)
+        assert rc == abi.GT_EINVAL and b"too deep" in ctx.lib.gt_last_error()
+    finally:
+        ctx.set_tuning(block_size=old.block_size, stack_lds=old.stack_lds)
+        buf.free()
