@@ -43,7 +43,11 @@ __device__ __forceinline__ float rcp_rn(float d) {  // 2^-96 <= |d| < 2^126
   const float q = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
   return __builtin_fmaf(__builtin_fmaf(-d, q, 1.0f), r, q);
 }
-// n / d, with rd = rcp_rn(d).
+// 1 / d for |d| >= 2^-96. The reciprocal of 2^126 and more is subnormal, which rcp_rn cannot make: then the whole
+// wave divides. (No ray of an ordinary scene gets there: one comparison and a branch not taken.)
+__device__ __forceinline__ bool beyond_rcp(float d) { return __ballot(!(fabsf(d) < 0x1p126f)) != 0ull; }
+__device__ __forceinline__ float reciprocal(float d) { return beyond_rcp(d) ? 1.0f / d : rcp_rn(d); }
+// n / d, with rd = reciprocal(d) (from |d| = 2^126 on rd has fewer bits and the quotient may be an ulp off).
 __device__ __forceinline__ float div_rn(float n, float d, float rd) {
   float q = n * rd;
   q = __builtin_fmaf(__builtin_fmaf(-d, q, n), rd, q);
@@ -332,7 +336,7 @@ __device__ __forceinline__ bool tri_hit(f3 v0, f3 e1, f3 e2, f3 o, f3 d, float t
   f3 pvec = cross(d, e2);
   float det = dot(e1, pvec);
   if (fabsf(det) < 1e-10f) return false;
-  float inv = rcp_rn(det);
+  float inv = reciprocal(det);
   f3 tvec = o - v0;
   float u = dot(tvec, pvec) * inv;
   if (!(u >= 0.f && u <= 1.f)) return false;
@@ -621,9 +625,10 @@ __device__ __forceinline__ RayPre ray_pre(f3 o, f3 d) {
   RayPre r;
   r.o = o;
   float dd[3] = {d.x, d.y, d.z};
+  const bool plain = beyond_rcp(fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fabsf(d.z)));
   for (int a = 0; a < 3; ++a) {
     bool par = fabsf(dd[a]) <= EPS;
-    r.inv[a] = par ? INF : rcp_rn(dd[a]);
+    r.inv[a] = par ? INF : plain ? 1.0f / dd[a] : rcp_rn(dd[a]);
     r.neg[a] = r.inv[a] < 0.f;
   }
   return r;
@@ -860,7 +865,7 @@ __device__ __forceinline__ void walk_begin(const DScene& sc, f3 o, f3 d, float t
   w.o = o;
   w.d = d;
   for (int a = 0; a < 3; ++a) w.inv[a] = rp.inv[a];
-  w.rdd = rcp_rn(len2(d));
+  w.rdd = reciprocal(len2(d));
   w.time = time;
   w.closest = INF;
   w.self = self;
@@ -945,7 +950,7 @@ __device__ __forceinline__ bool walk_test(const GPrim* __restrict__ prims, uint3
     const f3 e1 = mk(p1.x, p1.y, p1.z), e2 = mk(p2.x, p2.y, p2.z);
     const f3 pvec = cross(w.d, e2);
     const float det = dot(e1, pvec);
-    const float inv = rcp_rn(det);
+    const float inv = reciprocal(det);
     const f3 tvec = w.o - mk(p0.x, p0.y, p0.z);
     const float u = dot(tvec, pvec) * inv;
     const f3 qvec = cross(tvec, e1);
