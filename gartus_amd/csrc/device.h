@@ -62,11 +62,7 @@ __device__ __forceinline__ float sqrt_rn(float x) {
   s = __builtin_fmaf(s, e, s);
   return __builtin_fmaf(__builtin_fmaf(-s, s, x), h, s);
 }
-__device__ __forceinline__ f3 operator/(f3 a, float s) {
-  if (!(fabsf(s) >= 0x1p-96f && fabsf(s) < 0x1p126f)) return {a.x / s, a.y / s, a.z / s};
-  const float r = rcp_rn(s);
-  return {div_rn(a.x, s, r), div_rn(a.y, s, r), div_rn(a.z, s, r)};
-}
+__device__ __forceinline__ f3 operator/(f3 a, float s) { return {a.x / s, a.y / s, a.z / s}; }
 constexpr float INV_PI = 1.0f / PI, INV_TAU = 1.0f / TAU;  // reciprocals for div_rn
 
 // n / d and n % d for n < 2^31 by a multiplication: mul = floor(2^shift / d) + 1 with
@@ -88,7 +84,11 @@ __device__ __forceinline__ float len2(f3 a) { return dot(a, a); }
 __device__ __forceinline__ f3 normalized(f3 a) {  // vector.rs:151-158
   float l = sqrt_rn(len2(a));
   if (l < EPS) return {0.f, 0.f, 0.f};
-  return a / l;
+  if (!(l < 0x1p126f)) return a / l;
+  // no component is larger than l, so only the sign of a zero is left to restore (div_rn makes +0 of -0); plain
+  // quotients here took the Cornell frame from 3.70 to 3.74 ms
+  const float r = rcp_rn(l);
+  return {copysignf(div_rn(a.x, l, r), a.x), copysignf(div_rn(a.y, l, r), a.y), copysignf(div_rn(a.z, l, r), a.z)};
 }
 __device__ __forceinline__ f3 reflected(f3 d, f3 n) { return d - 2.0f * dot(d, n) * n; }  // vector.rs:162
 __device__ __forceinline__ f3 refracted(f3 d, f3 n, float eta) {  // vector.rs:168-173

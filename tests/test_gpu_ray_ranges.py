@@ -79,3 +79,14 @@ def test_renders_with_directions_whose_square_is_beyond_the_reciprocals_range():
     camera.raw = c
     px = api.PathTracer(camera).render_hdr_image(scene).pixels
     np.testing.assert_array_equal(px, 0.0)
+
+
+def test_the_sign_of_zero_survives_a_normal():
+    """A sphere's u at the seam (outward = (-1, 0, -0)) is atan2 of a signed zero: 1, not 0."""
+    data = _scene(SPHERE, [[0.0, 0.0, 0.0, 1.0]], GREY)
+    o = np.array([[-5.0, 0.0, -0.0], [-5.0, 0.0, 0.0]], np.float32)
+    d = np.array([[1.0, 0.0, -0.0], [1.0, 0.0, 0.0]], np.float32)
+    got = _agrees_with_oracle(data, o, d)
+    ref = cpu_ref.Scene(data).intersect(o, d)
+    np.testing.assert_allclose(got["u"], ref["u"], rtol=0, atol=1e-6)
+    np.testing.assert_array_equal(got["u"], np.float32([1.0, 0.0]))
