@@ -1090,10 +1090,9 @@ void zero_acc(const Launch& l, double4* acc, size_t n) {
 template <bool COUNT, bool MULTI, bool CAMERA, bool WIDE>
 static void launch_extend(const Launch& l, const Work& w, const Queues& q, uint32_t bounce) {
   const size_t lds = extend_lds_bytes(l.block, q.stack_cap);
-  static const hipError_t attr =  // once per instantiation: blocks of 1024 threads take more than 64 KiB
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&k_extend<COUNT, MULTI, CAMERA, WIDE>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-  (void)attr;
+  if (lds > 64 * 1024)  // large blocks: the limit is the device's own, so it is set for the one this launch goes to
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_extend<COUNT, MULTI, CAMERA, WIDE>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));  // a failure fails the launch
   hipLaunchKernelGGL((k_extend<COUNT, MULTI, CAMERA, WIDE>), dim3(l.grid), dim3(l.block), lds, l.stream,
                      Args{w.f, w.bt, q, bounce});
 }

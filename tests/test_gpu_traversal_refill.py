@@ -98,3 +98,26 @@ def test_odd_images_and_skies_match_oracle(w, h, ew, eh):
     g, r = gpu.pixels.reshape(-1, 3).astype(np.float64), ref.reshape(-1, 3)
     close = np.all(np.abs(g - r) <= 1e-3 * (1.0 + np.abs(r)), axis=1)
     assert close.mean() >= (1.0 if len(r) == 1 else 0.97), close.mean()
+
+
+def test_large_blocks_on_every_device():
+    """Blocks of 1024 threads take more LDS than a kernel gets unasked. The limit belongs to a device, so each
+    device's first context renders with them, eagerly and from a captured graph, after device 0's has. (With one
+    device the second context only shows that nothing is tied to the first.)"""
+    import torch
+    data, _, spec = scenes.cornell()
+    spec.pop("grid")
+    cam = _camera(dict(spec, spp=2), 65, 33)
+    devices = list(range(torch.cuda.device_count()))
+    images = []
+    for dev in devices if len(devices) > 1 else devices * 2:
+        ctx = api.Context(dev)
+        scene = api.RayScene(data, ctx).with_bvh()
+        tracer = api.PathTracer(cam)
+        images.append(tracer._render(scene, cam, None, None).pixels)
+        ctx.set_tuning(block_size=1024)
+        images += [tracer._render(scene, cam, None, None).pixels for _ in range(4)]
+        scene.close()
+        ctx.close()
+    for image in images[1:]:
+        np.testing.assert_array_equal(image, images[0])
