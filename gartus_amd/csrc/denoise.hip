@@ -12,6 +12,7 @@
 // Accumulation is fp32; weight gradients are summed per split and reduced
 // in a fixed order, so training steps are deterministic.
 #include "denoise.h"
+#include "rows_plan.h"
 
 #include <algorithm>
 #include <atomic>
@@ -1303,7 +1304,7 @@ bool launch_rows_all(hipStream_t s, RowsJob q, RowsMode mode) {
 // The layers that take the row kernel; false for the others, which take k_conv. Measured on one MI355X (us; k_conv or
 // the persistent LDS kernel that stood here before, then this one) on a 1920x1080 frame: 16->32 58 and 54, 32->32 76
 // and 54, 32->48 39 and 29, 48->48 47 and 32, 48->64 32 and 13, 64->64 34 and 22, 64->96 18 and 15, 96->96 22 and 15,
-// 48+32->32 171 and 117, 64+48->48 87 and 53, 96+64->64 62 and 45, the output 52 and 45. Where it lost, the layers stay
+// 48+32->32 171 and 117, 64+48->48 87 and 53, 96+64->64 62 and 45, the output 52 and 45, 80->32 179 and 113 (228 with k_conv). Where it lost, the layers stay
 // with k_conv: 128 channels and more in a part (128->128: 14 and 20; a wave's weights fill its registers for a few rows'
 // work). An instance takes as many output channels per wave as its registers hold, which divides the fragment loads by
 // them; the widest keep weights in LDS, and one wave per SIMD beat two that spill.
@@ -1320,20 +1321,29 @@ bool launch_rows(hipStream_t s, const RowsJob& q, int ca, int cb, RowsMode mode)
     return mode == ROWS_F32 ? launch_rows_nt<0, 32, true, 1, ROWS_F32, RowsCfg<2, 2>>(s, r)
                             : launch_rows_nt<0, 32, true, 1, ROWS_RADIANCE, RowsCfg<2, 2>>(s, r);
   }
+  const int nt = rows_frags(ca, cb, q.cout, mode == ROWS_GRAD || mode == ROWS_GRAD_MASK);
+  if (nt == 0) return false;
   switch (ca * 1000 + cb) {
     case 16: return launch_rows_all<0, 16, true, 2, RowsCfg<4, 1>>(s, q, mode);
     case 32:
-      if (q.cout == 48) return launch_rows_all<0, 32, true, 3, RowsCfg<2, 2>>(s, q, mode);
+      if (nt == 3) return launch_rows_all<0, 32, true, 3, RowsCfg<2, 2>>(s, q, mode);
       if (q.cout == 32) return launch_rows_all<0, 32, true, 2, RowsCfg<2, 2>>(s, q, mode);
       // five fragments a wave where they divide: 32->80 in one launch, 66 us at 16x256x256; 61 + 51 in launches of 2 and 1
-      if (q.cout % 80 == 0) return launch_rows_all<0, 32, false, 5, RowsCfg<1, 2>>(s, q, mode);
+      if (nt == 5) return launch_rows_all<0, 32, false, 5, RowsCfg<1, 2>>(s, q, mode);
       return launch_rows_all<0, 32, false, 2, RowsCfg<2, 2>>(s, q, mode);
     case 48:
-      if (q.cout == 48) return launch_rows_all<0, 48, true, 3, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
+      if (nt == 3) return launch_rows_all<0, 48, true, 3, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
       return launch_rows_all<0, 48, false, 2, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
     case 64: return launch_rows_all<0, 64, false, 2, RowsCfg<1, 1>, RowsCfg<2, 1>>(s, q, mode);
+    case 80: {  // an encoder level's first layer
+      if (mode != ROWS_FWD) return false;
+      RowsJob r = q;
+      r.groups = 1;
+      r.co_first = 0;
+      return launch_rows_nt<0, 80, false, 2, ROWS_FWD, RowsCfg<1, 1>>(s, r);
+    }
     case 96: return launch_rows_all<0, 96, false, 2, RowsCfg<1, 1>>(s, q, mode);
-    case 48032: return q.cout == 32 && launch_rows_all<48, 32, true, 2, RowsCfg<1, 1>, RowsCfg<1, 2>>(s, q, mode);
+    case 48032: return launch_rows_all<48, 32, true, 2, RowsCfg<1, 1>, RowsCfg<1, 2>>(s, q, mode);
     case 64032: return launch_rows_all<64, 32, false, 2, RowsCfg<1, 1>>(s, q, mode);
     case 64048: return launch_rows_all<64, 48, false, 3, RowsCfg<1, 1, 12>>(s, q, mode);
     case 96064: return launch_rows_all<96, 64, false, 2, RowsCfg<1, 1, 26>>(s, q, mode);

@@ -109,7 +109,7 @@ def test_forward_and_gradients_match_oracle(gpu_context, levels, channels, n, h,
 @pytest.mark.parametrize("levels,channels,n,h,w", [
     (2, (32, 48), 1, 2, 2), (2, (32, 48), 3, 17, 15), (2, (32, 64), 1, 6, 130), (2, (48, 64), 1, 66, 18),
     (2, (48, 64), 1, 64, 260), (2, (64, 96), 2, 10, 34), (2, (96, 128), 1, 5, 33), (2, (96, 128), 1, 131, 16),
-    (2, (32, 80), 1, 36, 34)])
+    (2, (32, 80), 1, 36, 34), (2, (80, 32), 1, 34, 70)])
 def test_row_kernel_shapes_match_oracle(gpu_context, levels, channels, n, h, w):
     _check_forward_and_gradients(gpu_context, levels, channels, n, h, w, abi.GT_DENOISE_LOSS_REL_L2)
 
