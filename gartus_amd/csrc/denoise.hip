@@ -1285,8 +1285,8 @@ bool launch_rows_mode(hipStream_t s, const RowsJob& q, RowsMode mode) {
   }
 }
 
-// The output channels in groups of NT fragments; a remainder of 1 to NT - 1 in a launch of its own.
-template <int CA, int CB, bool PAIRS, int NT, class CFG, class CFG1 = CFG, class CFG2 = CFG>
+// The output channels in groups of two fragments; an odd one in a launch of its own.
+template <int CA, int CB, bool PAIRS, int NT, class CFG, class CFG1 = CFG>
 bool launch_rows_all(hipStream_t s, RowsJob q, RowsMode mode) {
   const int frags = q.cout / 16, full = frags / NT, rest = frags % NT;
   q.groups = full;
@@ -1294,20 +1294,25 @@ bool launch_rows_all(hipStream_t s, RowsJob q, RowsMode mode) {
   if (full && !launch_rows_mode<CA, CB, PAIRS, NT, CFG>(s, q, mode)) return false;
   q.groups = 1;
   q.co_first = full * NT * 16;
-  if constexpr (NT > 1)
-    if (rest == 1) return launch_rows_mode<CA, CB, PAIRS, 1, CFG1>(s, q, mode);
-  if constexpr (NT > 2)
-    if (rest == 2) return launch_rows_mode<CA, CB, PAIRS, 2, CFG2>(s, q, mode);
-  return true;
+  return rest == 0 || launch_rows_mode<CA, CB, PAIRS, 1, CFG1>(s, q, mode);
 }
 
-// The layers that take the row kernel; false for the others, which take k_conv. Measured on one MI355X (us; k_conv or
-// the persistent LDS kernel that stood here before, then this one) on a 1920x1080 frame: 16->32 58 and 54, 32->32 76
-// and 54, 32->48 39 and 29, 48->48 47 and 32, 48->64 32 and 13, 64->64 34 and 22, 64->96 18 and 15, 96->96 22 and 15,
-// 48+32->32 171 and 117, 64+48->48 87 and 53, 96+64->64 62 and 45, the output 52 and 45, 80->32 179 and 113 (228 with k_conv). Where it lost, the layers stay
-// with k_conv: 128 channels and more in a part (128->128: 14 and 20; a wave's weights fill its registers for a few rows'
-// work). An instance takes as many output channels per wave as its registers hold, which divides the fragment loads by
-// them; the widest keep weights in LDS, and one wave per SIMD beat two that spill.
+// ... of a layer whose output channels are whole groups.
+template <int CA, int CB, bool PAIRS, int NT, class CFG>
+bool launch_rows_fit(hipStream_t s, RowsJob q, RowsMode mode) {
+  q.groups = q.cout / 16 / NT;
+  q.co_first = 0;
+  return launch_rows_mode<CA, CB, PAIRS, NT, CFG>(s, q, mode);
+}
+
+// The layers that take the row kernel (rows_frags); false for the others, which take k_conv. Measured on one MI355X (us;
+// k_conv or the persistent LDS kernel that stood here before, then this one) on a 1920x1080 frame: 16->32 58 and 54,
+// 32->32 76 and 54, 32->48 39 and 29, 48->48 47 and 32, 48->64 32 and 13, 64->64 34 and 22, 64->96 18 and 15, 96->96 22
+// and 15, 48+32->32 171 and 117, 64+48->48 87 and 53, 96+64->64 62 and 45, the output 52 and 45, 80->32 179 and 107 (228
+// with k_conv). 128 channels in a part lost and have no instance (128->128: 14 and 20; a wave's weights fill its registers
+// for a few rows' work). Parts of 80 and 112 channels (but for 80->32) and the other concatenations have none either: no
+// one has been built or measured. An instance takes as many output channels per wave as its registers hold, which divides
+// the fragment loads by them; the widest keep weights in LDS, and one wave per SIMD beat two that spill.
 //
 // PAIRS follows the layer, in the forward direction, so that a layer's sums are the same whatever kernel makes them:
 // taps pair over 16 channels in the shapes of the default network's full-resolution level and of level 1's 32->48 and
@@ -1321,20 +1326,25 @@ bool launch_rows(hipStream_t s, const RowsJob& q, int ca, int cb, RowsMode mode)
     return mode == ROWS_F32 ? launch_rows_nt<0, 32, true, 1, ROWS_F32, RowsCfg<2, 2>>(s, r)
                             : launch_rows_nt<0, 32, true, 1, ROWS_RADIANCE, RowsCfg<2, 2>>(s, r);
   }
-  const int nt = rows_frags(ca, cb, q.cout, mode == ROWS_GRAD || mode == ROWS_GRAD_MASK);
+  const int64_t tiles = int64_t(q.N) * ((q.H + kTR - 1) / kTR) * ((q.W + kTC - 1) / kTC);
+  const int nt = rows_frags(ca, cb, q.cout, mode == ROWS_GRAD || mode == ROWS_GRAD_MASK, tiles);
   if (nt == 0) return false;
   switch (ca * 1000 + cb) {
-    case 16: return launch_rows_all<0, 16, true, 2, RowsCfg<4, 1>>(s, q, mode);
+    case 16:
+      if (nt == 3) return launch_rows_fit<0, 16, true, 3, RowsCfg<2, 2>>(s, q, mode);
+      return launch_rows_all<0, 16, true, 2, RowsCfg<4, 1>>(s, q, mode);
     case 32:
-      if (nt == 3) return launch_rows_all<0, 32, true, 3, RowsCfg<2, 2>>(s, q, mode);
-      if (q.cout == 32) return launch_rows_all<0, 32, true, 2, RowsCfg<2, 2>>(s, q, mode);
+      if (nt == 3) return launch_rows_fit<0, 32, true, 3, RowsCfg<2, 2>>(s, q, mode);
+      if (q.cout == 32) return launch_rows_fit<0, 32, true, 2, RowsCfg<2, 2>>(s, q, mode);
       // five fragments a wave where they divide: 32->80 in one launch, 66 us at 16x256x256; 61 + 51 in launches of 2 and 1
-      if (nt == 5) return launch_rows_all<0, 32, false, 5, RowsCfg<1, 2>>(s, q, mode);
+      if (nt == 5) return launch_rows_fit<0, 32, false, 5, RowsCfg<1, 2>>(s, q, mode);
       return launch_rows_all<0, 32, false, 2, RowsCfg<2, 2>>(s, q, mode);
     case 48:
-      if (nt == 3) return launch_rows_all<0, 48, true, 3, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
+      if (nt == 3) return launch_rows_fit<0, 48, true, 3, RowsCfg<1, 2>>(s, q, mode);
       return launch_rows_all<0, 48, false, 2, RowsCfg<1, 2>, RowsCfg<2, 1>>(s, q, mode);
-    case 64: return launch_rows_all<0, 64, false, 2, RowsCfg<1, 1>, RowsCfg<2, 1>>(s, q, mode);
+    case 64:
+      if (nt == 3) return launch_rows_fit<0, 64, false, 3, RowsCfg<1, 1>>(s, q, mode);
+      return launch_rows_all<0, 64, false, 2, RowsCfg<1, 1>, RowsCfg<2, 1>>(s, q, mode);
     case 80: {  // an encoder level's first layer
       if (mode != ROWS_FWD) return false;
       RowsJob r = q;
@@ -1342,11 +1352,13 @@ bool launch_rows(hipStream_t s, const RowsJob& q, int ca, int cb, RowsMode mode)
       r.co_first = 0;
       return launch_rows_nt<0, 80, false, 2, ROWS_FWD, RowsCfg<1, 1>>(s, r);
     }
-    case 96: return launch_rows_all<0, 96, false, 2, RowsCfg<1, 1>>(s, q, mode);
-    case 48032: return launch_rows_all<48, 32, true, 2, RowsCfg<1, 1>, RowsCfg<1, 2>>(s, q, mode);
-    case 64032: return launch_rows_all<64, 32, false, 2, RowsCfg<1, 1>>(s, q, mode);
-    case 64048: return launch_rows_all<64, 48, false, 3, RowsCfg<1, 1, 12>>(s, q, mode);
-    case 96064: return launch_rows_all<96, 64, false, 2, RowsCfg<1, 1, 26>>(s, q, mode);
+    case 96:
+      if (nt == 3) return launch_rows_fit<0, 96, false, 3, RowsCfg<1, 1, 6>>(s, q, mode);
+      return launch_rows_all<0, 96, false, 2, RowsCfg<1, 1>>(s, q, mode);
+    case 48032: return launch_rows_fit<48, 32, true, 2, RowsCfg<1, 1>>(s, q, mode);
+    case 64032: return launch_rows_fit<64, 32, false, 2, RowsCfg<1, 1>>(s, q, mode);
+    case 64048: return launch_rows_fit<64, 48, false, 3, RowsCfg<1, 1, 12>>(s, q, mode);
+    case 96064: return launch_rows_fit<96, 64, false, 2, RowsCfg<1, 1, 26>>(s, q, mode);
     default: return false;
   }
 }
@@ -1364,10 +1376,8 @@ void launch_groups(hipStream_t s, int nt, int first_frag, int groups, const uint
   }
 }
 
-// Output channels in groups of NT 16-channel fragments, then one launch for
-// the rest. Levels with few tiles take narrower groups (more blocks, each
-// staging the same halo for fewer channels), so that the launch still has
-// blocks for most CUs.
+// The row kernel for the layers it takes. Otherwise output channels in groups
+// of NT 16-channel fragments (conv_frags), then one launch for the rest.
 template <bool DGRAD, bool F32>
 void launch_conv(hipStream_t s, const uint16_t* x, const uint16_t* mask, int cin, const uint16_t* xa, int ca,
                  const uint16_t* w, const float* bias, void* y, int cout, Dims d, int relu,
@@ -1381,7 +1391,7 @@ void launch_conv(hipStream_t s, const uint16_t* x, const uint16_t* mask, int cin
     if (like && launch_rows(s, q, xa ? ca : 0, xa ? cin - ca : cin, mode)) return;
   }
   const int tiles = d.n * ((d.h + kTR - 1) / kTR) * ((d.w + kTC - 1) / kTC);
-  const int nt = tiles >= 1024 ? 4 : tiles >= 256 ? 2 : 1;
+  const int nt = conv_frags(tiles);
   const int frags = cout / 16, full = frags / nt, rest = frags % nt;
   if (full) launch_groups<DGRAD, F32>(s, nt, 0, full, x, mask, cin, xa, ca, w, bias, y, cout, d, relu, pooled, omask);
   if (rest)

@@ -2,4 +2,6 @@
 // Built by tests/test_rows_plan.py with g++.
 #include "../gartus_amd/csrc/rows_plan.h"
 
-extern "C" int shim_rows_frags(int ca, int cb, int cout, int grad) { return gdn::rows_frags(ca, cb, cout, grad != 0); }
+extern "C" int shim_rows_frags(int ca, int cb, int cout, int grad, int64_t tiles) {
+  return gdn::rows_frags(ca, cb, cout, grad != 0, tiles);
+}

@@ -14,11 +14,55 @@ def shim(tmp_path_factory):
     out = tmp_path_factory.mktemp("shim") / "librowsplan.so"
     subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-o", str(out),
                     str(ROOT / "tests" / "rows_plan_shim.cpp")], check=True)
-    return C.CDLL(str(out))
+    lib = C.CDLL(str(out))
+    lib.shim_rows_frags.argtypes = [C.c_int] * 4 + [C.c_int64]
+    return lib
+
+
+def _frags(shim, ca, cb, cout, grad, n, h, w):
+    return shim.shim_rows_frags(ca, cb, cout, int(grad), n * -(-h // 4) * -(-w // 64))
 
 
 def test_an_encoder_layer_of_80_to_32_takes_the_row_kernel(shim):
     """k_conv takes twice as long on it at 1920x1080. Only that forward layer has an instance of 80 channels."""
-    assert shim.shim_rows_frags(0, 80, 32, 0) == 2
-    assert shim.shim_rows_frags(0, 80, 32, 1) == 0
-    assert all(shim.shim_rows_frags(0, 80, c, 0) == 0 for c in (16, 48, 64, 80, 96, 112, 128))
+    for size in ((1, 8, 12), (1, 1080, 1920)):
+        assert _frags(shim, 0, 80, 32, False, *size) == 2
+        assert _frags(shim, 0, 80, 32, True, *size) == 0
+        assert all(_frags(shim, 0, 80, c, False, *size) == 0 for c in (16, 48, 64, 80, 96, 112, 128))
+
+
+@pytest.mark.parametrize("grad", [False, True], ids=["forward", "gradient"])
+def test_small_images_take_the_faster_kernel(shim, grad):
+    """Forward layers of 64 channels, and layers whose output channels need a second launch, stay with k_conv on
+    images where it is faster; the others, and all of them on a 1920x1080 frame, take the row kernel."""
+    for cin, couts in ((64, (48, 80, 112) if grad else (32, 48, 64, 80, 96, 112, 128)), (16, (80, 112)), (32, (80, 112)), (48, (80, 112)),
+                       (96, (48, 80, 112))):
+        for cout in couts:
+            assert _frags(shim, 0, cin, cout, grad, 1, 32, 48) == 0, (cin, cout)
+            assert _frags(shim, 0, cin, cout, grad, 1, 1080, 1920) > 0, (cin, cout)
+    for cin, couts in ((16, (16, 32, 48, 64, 96, 128)), (32, (16, 32, 48, 64, 96, 128)), (48, (16, 32, 48, 64, 96, 128)),
+                       (64, (16, 32, 64, 96, 128) if grad else (16,)), (96, (16, 32, 64, 96, 128))):
+        for cout in couts:
+            assert _frags(shim, 0, cin, cout, grad, 1, 2, 2) > 0, (cin, cout)
+
+
+def test_lines_between_the_kernels_follow_k_convs_blocks(shim):
+    """The same layer on both sides of its line, where k_conv changes its groups too (256 tiles)."""
+    assert _frags(shim, 0, 64, 64, False, 1, 128, 128) == 0 and _frags(shim, 0, 64, 64, False, 1, 200, 256) == 2
+    assert _frags(shim, 0, 64, 32, False, 1, 256, 384) == 0 and _frags(shim, 0, 64, 32, False, 1, 360, 640) == 2
+    assert _frags(shim, 0, 64, 112, True, 1, 256, 256) == 0 and _frags(shim, 0, 64, 112, True, 1, 256, 384) == 2
+    assert [_frags(shim, 0, 64, 16, False, 1, h, w) for h, w in ((128, 128), (200, 256), (360, 640))] == [2, 0, 2]
+
+
+@pytest.mark.parametrize("cin", [16, 32, 48, 64, 96])
+def test_48_output_channels_are_one_launch(shim, cin):
+    """In groups of two fragments and one, the input was read twice: slower than k_conv on large images."""
+    assert _frags(shim, 0, cin, 48, False, 1, 1080, 1920) == _frags(shim, 0, cin, 48, True, 16, 256, 256) == 3
+
+
+def test_concatenations_with_an_instance(shim):
+    """A decoder layer has as many output channels as its skip part."""
+    for ca, cb in ((48, 32), (64, 32), (64, 48), (96, 64)):
+        assert [c for c in range(16, 129, 16) if _frags(shim, ca, cb, c, False, 1, 1080, 1920)] == [cb]
+    for ca, cb in ((32, 16), (96, 32), (80, 48), (128, 96), (112, 80)):
+        assert _frags(shim, ca, cb, cb, False, 1, 1080, 1920) == 0
