@@ -1253,24 +1253,13 @@ struct RowsCfg {
 
 template <int CA, int CB, bool PAIRS, int NT, RowsMode MODE, class CFG>
 bool launch_rows_nt(hipStream_t s, RowsJob q) {
-  const int waves = device_cus() * 4 * CFG::WAVES;
-  q.nstrip = (q.W + 15) / 16;
-  // rows per segment: the fewest rows in sequence, each segment costing two rows more than it makes
-  int best = 0;
-  int64_t best_cost = INT64_MAX;
-  for (int r : {64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
-    const int64_t jobs = int64_t(q.N) * ((q.H + r - 1) / r) * q.nstrip * q.groups;
-    const int64_t cost = (jobs + waves - 1) / waves * (std::min(r, q.H) + 2);
-    if (cost < best_cost) best = r, best_cost = cost;
-  }
+  const RowsSplit p = rows_split(q.N, q.H, q.W, q.groups, device_cus() * 4 * CFG::WAVES);
   const size_t widest = std::max({CA * 2, CB * 2, q.cout * (MODE == ROWS_F32 ? 4 : 2), 12});
-  if (size_t(best + 2) * q.W * widest >= kRowsBytes) return false;
-  q.seg_rows = best;
-  q.nseg = (q.H + best - 1) / best;
-  const int64_t quads = (int64_t(q.N) * q.nseg * q.nstrip + 31) / 32 * q.groups;  // blocks an XCD could use
-  int bpx = int(std::min<int64_t>(quads, std::max(waves / 32, q.groups)));
-  bpx = std::max(bpx / q.groups, 1) * q.groups;
-  hipLaunchKernelGGL((k_conv_rows<CA, CB, PAIRS, NT, MODE, CFG::WAVES, CFG::PF, CFG::LDSA>), dim3(8 * bpx), dim3(256), 0, s, q);
+  if (size_t(p.rows + 2) * q.W * widest >= kRowsBytes) return false;
+  q.seg_rows = p.rows;
+  q.nseg = p.segs;
+  q.nstrip = p.strips;
+  hipLaunchKernelGGL((k_conv_rows<CA, CB, PAIRS, NT, MODE, CFG::WAVES, CFG::PF, CFG::LDSA>), dim3(8 * p.blocks), dim3(256), 0, s, q);
   return true;
 }
 

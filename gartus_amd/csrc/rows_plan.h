@@ -1,5 +1,6 @@
-// rows_plan.h — which convolution layers the row kernel (denoise.hip) takes. Host code only.
+// rows_plan.h — which convolution layers the row kernel (denoise.hip) takes, and how it splits them. Host code only.
 #pragma once
+#include <algorithm>
 #include <cstdint>
 
 namespace gdn {
@@ -60,6 +61,28 @@ inline int rows_frags(int ca, int cb, int cout, bool grad, int64_t tiles) {
     case 96064: return cout == 64 ? 2 : 0;
     default: return 0;
   }
+}
+
+// A launch of the row kernel: n images of h x w in segments of `rows` rows (the last one shorter) by strips of 16
+// columns, for `groups` groups of output channels, on a chip that holds `waves` waves.
+struct RowsSplit {
+  int rows, segs, strips;
+  int blocks;  // of each of the 8 XCDs, a multiple of groups; a block's four waves take a tile (segment x strip) each
+};
+inline RowsSplit rows_split(int n, int h, int w, int groups, int waves) {
+  RowsSplit s{0, 0, (w + 15) / 16, 0};
+  // the fewest rows in sequence, each segment costing two rows more than it makes
+  int64_t best = INT64_MAX;
+  for (int r : {64, 48, 32, 24, 16, 12, 8, 6, 4, 2}) {
+    const int64_t jobs = int64_t(n) * ((h + r - 1) / r) * s.strips * groups;
+    const int64_t cost = (jobs + waves - 1) / waves * (std::min(r, h) + 2);
+    if (cost < best) s.rows = r, best = cost;
+  }
+  s.segs = (h + s.rows - 1) / s.rows;
+  const int64_t quads = (int64_t(n) * s.segs * s.strips + 31) / 32 * groups;  // blocks an XCD could use
+  const int bpx = int(std::min<int64_t>(quads, std::max(waves / 32, groups)));
+  s.blocks = std::max(bpx / groups, 1) * groups;
+  return s;
 }
 
 }  // namespace gdn

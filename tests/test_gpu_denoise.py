@@ -103,9 +103,10 @@ def test_forward_and_gradients_match_oracle(gpu_context, levels, channels, n, h,
     _check_forward_and_gradients(gpu_context, levels, channels, n, h, w, loss)
 
 
-# Every channel pair with a row-kernel instance (strips of 16 columns, segments of 2 to 64 rows, output
-# channels in groups of 16 to 48 and a remainder), forward and backward, at widths below, at and beyond a
-# strip, heights of one and several segments, and more strips than a block's four waves.
+# Channel pairs of the row kernel's instances and of the layers beside them, forward and backward, at widths below, at
+# and beyond a strip of 16 columns and more strips than a block's four waves. These images are small: the launches have
+# segments of 1 to 8 rows, one a wave, and the layers that take k_conv on small images (rows_frags) take it here. Longer
+# segments and several of them a wave: test_long_segments_match_single_images.
 @pytest.mark.parametrize("levels,channels,n,h,w", [
     (2, (32, 48), 1, 2, 2), (2, (32, 48), 3, 17, 15), (2, (32, 64), 1, 6, 130), (2, (48, 64), 1, 66, 18),
     (2, (48, 64), 1, 64, 260), (2, (64, 96), 2, 10, 34), (2, (96, 128), 1, 5, 33), (2, (96, 128), 1, 131, 16),
@@ -114,11 +115,11 @@ def test_row_kernel_shapes_match_oracle(gpu_context, levels, channels, n, h, w):
     _check_forward_and_gradients(gpu_context, levels, channels, n, h, w, abi.GT_DENOISE_LOSS_REL_L2)
 
 
-# The gradient of the decoder's concatenation, 80 channels from 32 or 112 from 48, is split over
-# launches of its output channels; 128 x 2048 at full resolution gives every wave several segments.
-# (The oracle takes about 20 and 50 s here.)
+# The gradient of the decoder's concatenation: 80 channels from 32 in one launch, 112 from 48 in one of six fragments
+# and one of the odd seventh, at a full resolution where every wave of the chip has a segment. (The oracle takes about
+# 20 and 50 s here.)
 @pytest.mark.parametrize("channels", [(32, 48), (48, 64)], ids=["cat80", "cat112"])
-def test_persistent_data_gradients_match_oracle(gpu_context, channels):
+def test_concatenation_gradients_match_oracle(gpu_context, channels):
     _check_forward_and_gradients(gpu_context, 2, channels, 1, 128, 2048, abi.GT_DENOISE_LOSS_REL_L2)
 
 
@@ -183,4 +184,46 @@ def test_halves_network_matches_oracle(gpu_context, levels, channels, n, h, w):
     assert rel < 0.01 * np.sqrt(len(net.convs)) and cos > 0.998, (rel, cos)  # the bar of the test above
     # the first convolution's gradient reaches the difference channels
     assert np.abs(gg.reshape(-1, 9, 16)[:, :, 9:12]).max() > 0
+    dn.close()
+
+
+# A batch of small images whose layers the row kernel walks in long segments, with a shorter last one, several tiles a
+# wave (test_rows_plan.py checks that it does).
+LONG_BATCH = (512, 132, 96)
+LONG_CHANNELS = [(16, 64), (32, 48), (32, 64), (32, 80), (32, 112), (48, 64), (48, 80), (48, 96), (64, 96), (64, 112),
+                 (80, 32), (96, 48), (96, 80), (96, 128), (112, 16)]
+
+
+@pytest.mark.parametrize("channels", LONG_CHANNELS, ids=lambda c: f"{c[0]}-{c[1]}")
+def test_long_segments_match_single_images(gpu_context, channels):
+    """A network's images do not depend on the batch they come in: bit for bit the images of a batch of one, whose
+    layers run in short segments or through k_conv and match the oracle above. The gradients are the mean of the single
+    ones (the batch's scale is a power of two): a data gradient sums in another order in k_conv, so that at most about
+    2^-9 of its bf16 values round the other way by 2^-8, 2^-8 * 2^-4.5 = 1.7e-4 of its norm a layer, over six layers in
+    a row below 2e-3; weight gradients sum in fp32 in another order, below 1e-4."""
+    import torch
+    n, h, w = LONG_BATCH
+    say(f"denoiser levels 2 channels {channels} batch {n}x{h}x{w}")
+    net, *images = _problem(2, channels, 4, h, w, seed=7)
+    dn = Denoiser(gpu_context, 2, channels, loss=abi.GT_DENOISE_LOSS_REL_L2)
+    dn.set_params(net.params.astype(np.float32))
+    one = [torch.from_numpy(x).cuda() for x in images]
+    many = [x.repeat(n // 4, 1, 1, 1) for x in one]
+    torch.cuda.synchronize()
+
+    singles = [dn.infer(*(x[k:k + 1] for x in one[:3])) for k in range(4)]
+    batch = dn.infer(*many[:3])
+    gpu_context.synchronize()
+    single = torch.cat(singles)
+    assert torch.isfinite(single).all() and single.std() > 0
+    assert torch.equal(batch.reshape(n // 4, 4, h, w, 3), single.expand(n // 4, 4, h, w, 3))
+
+    parts = [dn.loss_and_gradients(*(x[k:k + 1] for x in one)) for k in range(4)]
+    loss, grads = dn.loss_and_gradients(*many)
+    assert loss == pytest.approx(np.mean([p[0] for p in parts]), rel=1e-5)
+    g, ref = np.asarray(grads, np.float64), np.mean([np.asarray(p[1], np.float64) for p in parts], axis=0)
+    for i, (cin, cout, _) in enumerate(net.convs):
+        w0, b0 = net.offsets[i]
+        rel = np.linalg.norm(g[w0:b0 + cout] - ref[w0:b0 + cout]) / np.linalg.norm(ref[w0:b0 + cout])
+        assert rel < 2e-3, f"conv {i} {cin}->{cout}: {rel:.2e}"
     dn.close()

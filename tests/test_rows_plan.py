@@ -1,10 +1,12 @@
-"""The host-side rules of the denoiser's row kernel (gartus_amd/csrc/rows_plan.h): which layers take it. CPU
-only: the rules are compiled with g++ through tests/rows_plan_shim.cpp."""
+"""The host-side rules of the denoiser's row kernel (gartus_amd/csrc/rows_plan.h): which layers take it, and
+how a launch is split. CPU only: the rules are compiled with g++ through tests/rows_plan_shim.cpp."""
 import ctypes as C
 import subprocess
 from pathlib import Path
 
 import pytest
+
+from test_gpu_denoise import LONG_BATCH
 
 ROOT = Path(__file__).resolve().parent.parent
 
@@ -66,3 +68,32 @@ def test_concatenations_with_an_instance(shim):
         assert [c for c in range(16, 129, 16) if _frags(shim, ca, cb, c, False, 1, 1080, 1920)] == [cb]
     for ca, cb in ((32, 16), (96, 32), (80, 48), (128, 96), (112, 80)):
         assert _frags(shim, ca, cb, cb, False, 1, 1080, 1920) == 0
+
+
+@pytest.mark.parametrize("level", [0, 1])
+@pytest.mark.parametrize("waves", [1024, 2048, 4096], ids=["1-wave", "2-waves", "4-waves"])
+def test_the_long_batch_reaches_every_part_of_the_walk(shim, level, waves):
+    """The batch of test_gpu_denoise.py's long segments, on 256 CUs of 1, 2 or 4 waves a SIMD, for every number of
+    output groups (four waves a SIMD: layers of 16 channels, four groups at most): several segments of more rows than
+    the fragment ring holds (at most five), a shorter last one, and waves that walk more than one tile."""
+    n, h, w = LONG_BATCH[0], LONG_BATCH[1] >> level, LONG_BATCH[2] >> level
+    out = (C.c_int * 4)()
+    for groups in range(1, 5 if waves == 4096 else 9):
+        shim.shim_rows_split(n, h, w, groups, waves, out)
+        rows, segs, strips, blocks = out
+        assert segs >= 2 and rows >= 12 and 0 < h - (segs - 1) * rows < rows, (groups, list(out))
+        if (level, waves, groups) != (1, 4096, 1):  # 16->16 and 16->32 below the full resolution: a tile a wave
+            tiles_at_once = 8 * 4 * (blocks // groups)
+            assert n * segs * strips > tiles_at_once, (groups, list(out))
+
+
+@pytest.mark.parametrize("n,h,w", [(1, 1, 1), (1, 2, 15), (1, 64, 16), (3, 17, 17), (1, 1088, 1920), (16, 256, 256),
+                                   (1, 4, 200000), (512, 2, 2)])
+def test_a_split_covers_the_image(shim, n, h, w):
+    out = (C.c_int * 4)()
+    for groups in (1, 2, 3, 7):
+        for waves in (1024, 4096):
+            shim.shim_rows_split(n, h, w, groups, waves, out)
+            rows, segs, strips, blocks = out
+            assert rows % 2 == 0 and (segs - 1) * rows < h <= segs * rows and (strips - 1) * 16 < w <= strips * 16
+            assert blocks % groups == 0 and 0 < blocks <= max(waves // 32, groups)
