@@ -93,6 +93,18 @@ def build_oracle(verbose: bool = False) -> Path:
     return oracle / "libcpu_ref.so"
 
 
+def build_math_probe(verbose: bool = False) -> Path:
+    """Compiles the device-arithmetic probe (test infrastructure) in-tree."""
+    out = ROOT / "tests" / "libdevice_math_probe.so"
+    tmp = out.with_suffix(".so.tmp")
+    _run([_hipcc(), *HIP_FLAGS, "-shared", "-o", str(tmp), str(ROOT / "tests" / "device_math_probe.hip")])
+    os.replace(tmp, out)
+    if verbose:
+        print(f"built {out}")
+    return out
+
+
 if __name__ == "__main__":
     build_library(verbose=True)
     build_oracle(verbose=True)
+    build_math_probe(verbose=True)

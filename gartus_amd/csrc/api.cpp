@@ -433,13 +433,6 @@ int make_camera(const gt_camera* c, GCamera* g) {
   return GT_OK;
 }
 
-// Div31 of d in [1, 2^31]: exact quotients of every n < 2^31.
-gtd::Div31 make_div31(uint32_t d) {
-  uint32_t l = 0;
-  while ((uint64_t(1) << l) < d) ++l;
-  return {d, uint32_t((uint64_t(1) << (31 + l)) / d + 1), 31 + l};
-}
-
 gtd::DScene device_scene(const gt_scene* s, uint32_t width) {
   gtd::DScene d;
   d.nodes2 = s->nodes2.p;
@@ -559,7 +552,7 @@ int make_frame(gt_context* ctx, const gt_scene* scene, const gt_camera* camera, 
     f->env.tex = env->tex.p; f->env.alias = env->alias.p;
     f->env.row_cos = env->row_cos.p;
     if (env->kind == 2) {
-      f->env.row = make_div31(env->w);
+      f->env.row = gtd::make_div31(env->w);
       f->env.inv_w = 1.0f / float(env->w);
     }
   }
@@ -569,7 +562,7 @@ int make_frame(gt_context* ctx, const gt_scene* scene, const gt_camera* camera, 
   f->npix = f->cam.width * f->cam.height;
   f->nact = f->npix;
   f->pixmap = nullptr;
-  f->by_width = make_div31(std::max(f->cam.width, 1u));
+  f->by_width = gtd::make_div31(std::max(f->cam.width, 1u));
   return GT_OK;
 }
 
@@ -692,7 +685,7 @@ int run_jobs(gt_context* ctx, std::vector<FrameJob>& jobs, bool multi, int out_i
   uint64_t off = 0;
   for (FrameJob& j : jobs) {
     j.f.acc = ctx->acc.p + off;
-    j.f.by_nact = make_div31(std::max(j.f.nact, 1u));
+    j.f.by_nact = gtd::make_div31(std::max(j.f.nact, 1u));
     off += j.f.npix;
   }
   size_t seg_total = 0;

@@ -26,16 +26,19 @@ __device__ __forceinline__ f3 operator-(f3 a, f3 b) { return {a.x - b.x, a.y - b
 __device__ __forceinline__ f3 operator-(f3 a) { return {-a.x, -a.y, -a.z}; }
 __device__ __forceinline__ f3 operator*(float s, f3 a) { return {s * a.x, s * a.y, s * a.z}; }
 __device__ __forceinline__ f3 operator*(f3 a, float s) { return {a.x * s, a.y * s, a.z * s}; }
-// Correctly rounded FP32 division and square root for operands whose results
-// and remainders stay in the normal range, as those of a traced ray do: the
-// compiler's general forms also scale their operands and handle zeros,
-// infinities and denormals, and cannot share one divisor's reciprocal. The
-// refinement steps are Markstein's (IBM J. Res. Dev. 34, 1990): with fma, a
+// Correctly rounded FP32 reciprocals, quotients and square roots for operands
+// whose results and remainders stay in the normal range, as those of a traced
+// ray do: the compiler's general forms also scale their operands and handle
+// zeros, infinities and denormals, and cannot share one divisor's reciprocal.
+// The refinement steps are Markstein's (IBM J. Res. Dev. 34, 1990): with fma, a
 // residual is exact, so a quotient or root within an ulp of the true value comes
-// out correctly rounded, the same bits as the operator. Vector instructions: 7
-// for a reciprocal, 5 for each further quotient of the same divisor and 8 for a
-// root, against about 10, 10 and 14. Together with straight-line primitive tests, a
-// sky lookup without fmod and table cosines, on one MI355X: 720p terrain 13.7 ->
+// out correctly rounded. The tests compare reciprocals and roots with the
+// operators over every operand of the ranges stated here, quotients over every
+// divisor with sampled numerators: the same bits, but that a zero quotient is
+// always +0 and an infinite numerator gives NaN. Vector instructions: 7 for a
+// reciprocal, 5 for each further quotient of the same divisor and 8 for a root,
+// against about 10, 10 and 14. Together with straight-line primitive tests, a sky
+// lookup without fmod and table cosines, on one MI355X: 720p terrain 13.7 ->
 // 13.1 ms, 12 small scenes 5.3 -> 5.0 ms, 1080p GGX/environment 13.1 -> 12.8 ms.
 __device__ __forceinline__ float rcp_rn(float d) {  // 2^-96 <= |d| < 2^126
   float r = __builtin_amdgcn_rcpf(d);
@@ -66,10 +69,16 @@ __device__ __forceinline__ f3 operator/(f3 a, float s) { return {a.x / s, a.y / 
 constexpr float INV_PI = 1.0f / PI, INV_TAU = 1.0f / TAU;  // reciprocals for div_rn
 
 // n / d and n % d for n < 2^31 by a multiplication: mul = floor(2^shift / d) + 1 with
-// shift = 31 + ceil(log2 d) (Granlund and Montgomery, PLDI 1994). Made on the host (make_div31).
+// shift = 31 + ceil(log2 d) (Granlund and Montgomery, PLDI 1994).
 struct Div31 {
   uint32_t d, mul, shift;
 };
+// Div31 of d in [1, 2^31].
+inline Div31 make_div31(uint32_t d) {
+  uint32_t l = 0;
+  while ((uint64_t(1) << l) < d) ++l;
+  return {d, uint32_t((uint64_t(1) << (31 + l)) / d + 1), 31 + l};
+}
 __device__ __forceinline__ uint32_t div31(uint32_t n, const Div31& k, uint32_t* rem) {
   const uint32_t q = uint32_t((uint64_t(n) * k.mul) >> k.shift);
   *rem = n - q * k.d;
