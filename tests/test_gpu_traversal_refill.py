@@ -4,6 +4,7 @@ and node width. Bit-exact comparisons: the paths are the same, so the images are
 """
 import numpy as np
 import pytest
+import torch  # before the library loads: one HIP runtime per process
 
 pytestmark = pytest.mark.gpu
 
@@ -104,7 +105,6 @@ def test_large_blocks_on_every_device():
     """Blocks of 1024 threads take more LDS than a kernel gets unasked. The limit belongs to a device, so each
     device's first context renders with them, eagerly and from a captured graph, after device 0's has. (With one
     device the second context only shows that nothing is tied to the first.)"""
-    import torch
     data, _, spec = scenes.cornell()
     spec.pop("grid")
     cam = _camera(dict(spec, spp=2), 65, 33)
