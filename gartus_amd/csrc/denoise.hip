@@ -50,7 +50,7 @@ constexpr int kTR = 4;               // tile rows, one per wave
 constexpr int kTC = 64;              // tile columns, 4 fragments of 16
 constexpr int kHR = kTR + 2, kHC = kTC + 2;
 constexpr int kCK = 32;              // input channels per staged chunk
-constexpr int kLS = kCK;             // LDS row (pixel or weight row) in bf16: 64 B, pieces swizzled by swz<2>
+constexpr int kLS = kCK;             // LDS row (pixel or weight row) in bf16: 64 B, pieces swizzled by swz
 
 // A 16-byte LDS read (ds_read_b128) is served 16 lanes at a time: lanes
 // 0-31 and 32-63 are separate halves, and within a half the quads (4 lanes)
@@ -58,16 +58,12 @@ constexpr int kLS = kCK;             // LDS row (pixel or weight row) in bf16: 6
 // in the next. Two lanes of a pass conflict when their addresses differ but
 // agree in bits 4-7 (the same four of the 64 banks). An MFMA operand read
 // takes pixels P .. P + 15 (lane & 15) of piece q = (lane >> 4) & 1 and, in
-// lanes 32-63, the next sub-slice. With 32-byte pixels (16 channels, G = 1)
-// every pass then covers the 16 bank groups once as they are; with 64-byte
-// pixels (G = 2) piece q of pixel p goes to slot q ^ swz<2>(p), and the
-// weight rows the same way by row. Both layouts were checked conflict free
-// against SQ_LDS_BANK_CONFLICT for every read of a chunk, mirrored taps and
-// 16-channel chunks in 64-byte rows included.
-template <int G>
-__device__ __forceinline__ int swz(int p) {
-  return G == 2 ? (p >> 1) & 3 : 0;
-}
+// lanes 32-63, the next sub-slice. In 64-byte rows piece q of pixel p goes to
+// slot q ^ swz(p), and the weight rows the same way by row: every pass then
+// covers the 16 bank groups once. The layout was checked conflict free against
+// SQ_LDS_BANK_CONFLICT for every read of a chunk, mirrored taps and 16-channel
+// chunks included.
+__device__ __forceinline__ int swz(int p) { return (p >> 1) & 3; }
 
 template <int NT>
 constexpr int conv_out_stride() {  // fp32 row stride of the output staging: the 4 lane groups' rows land in distinct banks
@@ -117,10 +113,10 @@ __device__ __forceinline__ void conv_chunk(const uint16_t* halo, const uint16_t*
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int r = tap * NT * 16 + j * 16 + col;
-      b[j] = valid ? *reinterpret_cast<const uint4*>(wts + r * kLS + 8 * (q ^ swz<2>(r))) : make_uint4(0, 0, 0, 0);
+      b[j] = valid ? *reinterpret_cast<const uint4*>(wts + r * kLS + 8 * (q ^ swz(r))) : make_uint4(0, 0, 0, 0);
     }
     const int p0 = (wave + 1 + dy) * kHC + col + 1 + dx;  // pixels p0 + 16 f share the swizzle of p0
-    const uint16_t* arow = halo + p0 * kLS + 8 * (q ^ swz<2>(p0));
+    const uint16_t* arow = halo + p0 * kLS + 8 * (q ^ swz(p0));
 #pragma unroll
     for (int f = 0; f < 4; ++f) {
       const uint4 a = valid ? *reinterpret_cast<const uint4*>(arow + f * 16 * kLS) : make_uint4(0, 0, 0, 0);
@@ -170,7 +166,7 @@ __device__ __forceinline__ void conv_stage(uint16_t* halo, uint16_t* wts, const 
 #pragma unroll
     for (int k = 0; k < HI; ++k) {
       const int i = tid + 256 * k;
-      if (i < HP) *reinterpret_cast<uint4*>(halo + (i / QP) * kLS + 8 * ((i % QP) ^ swz<2>(i / QP))) = hv[k];
+      if (i < HP) *reinterpret_cast<uint4*>(halo + (i / QP) * kLS + 8 * ((i % QP) ^ swz(i / QP))) = hv[k];
     }
   }
   __builtin_amdgcn_sched_barrier(0);  // keep the two batches apart: fewer live registers
@@ -188,7 +184,7 @@ __device__ __forceinline__ void conv_stage(uint16_t* halo, uint16_t* wts, const 
 #pragma unroll
     for (int k = 0; k < WI; ++k) {
       const int i = tid + 256 * k;
-      if (i < WP) *reinterpret_cast<uint4*>(wts + (i / QP) * kLS + 8 * ((i % QP) ^ swz<2>(i / QP))) = wv[k];
+      if (i < WP) *reinterpret_cast<uint4*>(wts + (i / QP) * kLS + 8 * ((i % QP) ^ swz(i / QP))) = wv[k];
     }
   }
 }
@@ -358,9 +354,12 @@ __device__ __forceinline__ void lds_copy16(const uint4* dst, i32x4 src, uint32_t
 // load and store is such a buffer access, so a row's body has no branch and the
 // waits for the loads in flight are exact; the loads run PF rows ahead.
 //
-// Sums are made in a fixed order, the same as k_conv's and as the persistent kernel's that this one replaced: by
-// groups of input channels, tap by tap within one. A group of 32 channels takes one K = 32 MFMA step per tap. A group
-// of 16 pairs taps (0,1), (2,3), (4,5), (6,7), (8,-) in the two halves of K. A part's odd 16 channels are such a group;
+// Sums are made in a fixed order: by groups of input channels, tap by tap within one. Forward that is
+// the order of the kernels this one replaced, k_conv's or (PAIRS) the persistent LDS kernel's, bit for bit. A data
+// gradient takes the pixel taps in that order, so its weight taps come last to first, where k_conv takes the weight taps
+// in order and mirrors the pixels: the same terms, rounded otherwise here and there (gradients of a small batch differ by
+// a relative 7e-5; their error against 64 bits is the same). A group of 32 channels takes one K = 32 MFMA step per tap.
+// A group of 16 pairs taps (0,1), (2,3), (4,5), (6,7), (8,-) in the two halves of K. A part's odd 16 channels are such a group;
 // with PAIRS all are. Its fragments, of row i, are the column taps F = (-1 | 0), G = (+1 | -1) and H = (0 | +1), and
 // output row r takes F(r-1), G(r-1) with the upper half of G(r), H(r), F(r+1), G(r+1) with zeros. Two groups side by
 // side are loaded as one of 32 channels, three contiguous loads a row, and their fragments made by exchanging register
@@ -1303,9 +1302,9 @@ bool launch_rows_fit(hipStream_t s, RowsJob q, RowsMode mode) {
 // one has been built or measured. An instance takes as many output channels per wave as its registers hold, which divides
 // the fragment loads by them; the widest keep weights in LDS, and one wave per SIMD beat two that spill.
 //
-// PAIRS follows the layer, in the forward direction, so that a layer's sums are the same whatever kernel makes them:
+// PAIRS follows the layer, in the forward direction, so that its images stay the bits of the kernel that made it before:
 // taps pair over 16 channels in the shapes of the default network's full-resolution level and of level 1's 32->48 and
-// 48->48, 32 channels to a tap elsewhere.
+// 48->48 (the persistent kernel's), 32 channels to a tap elsewhere (k_conv's). Data gradients never pair.
 bool launch_rows(hipStream_t s, const RowsJob& q, int ca, int cb, RowsMode mode) {
   if (mode == ROWS_F32 || mode == ROWS_RADIANCE) {
     if (ca || cb != 32 || q.cout != 16) return false;

@@ -315,27 +315,17 @@ __device__ __forceinline__ uint32_t meta_of(const float4& p0) { return __float_a
 // hit_sphere_in_interval (object.rs:986-1013). The discriminant uses the
 // perpendicular-distance form a*(r^2 - |oc - (h/a) d|^2), algebraically equal
 // to h^2 - a*c and free of its cancellation in FP32.
-//
-// from_surface: the ray starts on this sphere (its origin is a hit on it).
-// In exact arithmetic one root is then 0 and the other 2h/a, so the sphere
-// is met again only by a ray heading inward, at the far root. FP32 cannot
-// place the origin on a large sphere within t_min (on the 1000-radius
-// ground sphere a coordinate's ulp is 6e-5 and the near root's error grows
-// as 1/cos at grazing angles), so the near root is skipped by this rule, not
-// compared with t_min: the decision the reference's f64 arithmetic makes.
-__device__ __forceinline__ bool sphere_hit(f3 c, float r, f3 o, f3 d, float tmin, float tmax, float* root,
-                                           bool from_surface = false) {
+__device__ __forceinline__ bool sphere_hit(f3 c, float r, f3 o, f3 d, float tmin, float tmax, float* root) {
   f3 oc = c - o;
   float a = len2(d);
   if (a <= EPS) return false;
   float h = dot(d, oc);
-  if (from_surface && h <= 0.f) return false;
   f3 perp = oc - (h / a) * d;
   float disc = a * (r * r - len2(perp));
   if (disc < 0.f) return false;
   float sq = sqrt_rn(disc);
   float first = (h - sq) / a;
-  if (!from_surface && tmin < first && first < tmax) { *root = first; return true; }
+  if (tmin < first && first < tmax) { *root = first; return true; }
   float second = (h + sq) / a;
   if (tmin < second && second < tmax) { *root = second; return true; }
   return false;
@@ -374,18 +364,13 @@ __device__ __forceinline__ bool quad_hit(f3 corner, f3 u, f3 v, f3 n, float inv_
   return true;
 }
 // One primitive record against a ray interval; returns the root only.
-// from_surface: the ray starts on this primitive. A ray leaving a plane
-// cannot meet it again (the reference's t is 0 up to rounding, below
-// t_min); a sphere is met again only at its far root (sphere_hit).
 __device__ __forceinline__ bool prim_test(const GPrim* __restrict__ prims, uint32_t k, f3 o, f3 d, float time,
-                                          float tmin, float tmax, PrimHit* h, uint32_t* meta_out,
-                                          bool from_surface) {
+                                          float tmin, float tmax, PrimHit* h, uint32_t* meta_out) {
   const float4* rec = reinterpret_cast<const float4*>(prims + k);
   float4 p0 = rec[0];
   uint32_t meta = meta_of(p0);
   *meta_out = meta;
   uint32_t kind = (meta >> GT_KIND_SHIFT) & GT_KIND_MASK;
-  if (from_surface && (kind == GK_TRIANGLE || kind == GK_QUAD)) return false;
   float4 p1 = rec[1];
   if (kind == GK_TRIANGLE) {
     float4 p2 = rec[2];
@@ -404,7 +389,7 @@ __device__ __forceinline__ bool prim_test(const GPrim* __restrict__ prims, uint3
     r = p1.w;
   }
   float root;
-  if (!sphere_hit(c, r, o, d, tmin, tmax, &root, from_surface)) return false;
+  if (!sphere_hit(c, r, o, d, tmin, tmax, &root)) return false;
   h->t = root; h->u = 0.f; h->v = 0.f;
   return true;
 }
@@ -664,12 +649,11 @@ __device__ __forceinline__ bool slab(const RayPre& r, float lox, float hix, floa
 // interval shrinking on each accepted hit (scene.rs:849-874).
 template <bool STATS>
 __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax,
-                                       uint32_t self, Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out,
-                                       Stats* stats, uint32_t* meta_out = nullptr) {
+                                       Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out, Stats* stats) {
   RayPre rp = ray_pre(o, d);
   float closest = tmax;
   bool any = false;
-  uint32_t best = 0, best_meta = 0;
+  uint32_t best = 0;
   PrimHit bh{0.f, 0.f, 0.f};
   if (STATS) { stats->node_tests += 1; }
   float root_entry;
@@ -688,10 +672,9 @@ __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time,
         PrimHit h;
         uint32_t meta;
         if (STATS) stats->candidates += 1;
-        if (prim_test(sc.prims, k, o, d, time, tmin, closest, &h, &meta, k == self)) {
+        if (prim_test(sc.prims, k, o, d, time, tmin, closest, &h, &meta)) {
           closest = h.t;
           best = k;
-          best_meta = meta;
           bh = h;
           any = true;
           leaf_hit = true;
@@ -739,7 +722,6 @@ __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time,
     *t_out = closest;
     *prim_out = best;
     if (hit_out) *hit_out = bh;
-    if (meta_out) *meta_out = best_meta;
   }
   return any;
 }
@@ -747,12 +729,11 @@ __device__ __forceinline__ bool trace2(const DScene& sc, f3 o, f3 d, float time,
 // Four-wide variant: children of a wide node are visited nearest-first.
 template <bool STATS>
 __device__ __forceinline__ bool trace4(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax,
-                                       uint32_t self, Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out,
-                                       Stats* stats, uint32_t* meta_out = nullptr) {
+                                       Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out, Stats* stats) {
   RayPre rp = ray_pre(o, d);
   float closest = tmax;
   bool any = false;
-  uint32_t best = 0, best_meta = 0;
+  uint32_t best = 0;
   PrimHit bh{0.f, 0.f, 0.f};
   float root_entry;
   if (STATS) stats->node_tests += 1;
@@ -771,8 +752,8 @@ __device__ __forceinline__ bool trace4(const DScene& sc, f3 o, f3 d, float time,
         PrimHit h;
         uint32_t meta;
         if (STATS) stats->candidates += 1;
-        if (prim_test(sc.prims, k, o, d, time, tmin, closest, &h, &meta, k == self)) {
-          closest = h.t; best = k; best_meta = meta; bh = h; any = true; leaf_hit = true;
+        if (prim_test(sc.prims, k, o, d, time, tmin, closest, &h, &meta)) {
+          closest = h.t; best = k; bh = h; any = true; leaf_hit = true;
         }
         if (meta & GT_LAST_BIT) break;
         ++k;
@@ -825,21 +806,15 @@ __device__ __forceinline__ bool trace4(const DScene& sc, f3 o, f3 d, float time,
     *t_out = closest;
     *prim_out = best;
     if (hit_out) *hit_out = bh;
-    if (meta_out) *meta_out = best_meta;
   }
   return any;
 }
 
-// self: the primitive (leaf order) the ray starts on, kNoSelf for a ray from
-// a camera or a caller; prim_test decides it by rule, not by t_min.
-constexpr uint32_t kNoSelf = 0xffffffffu;
 template <bool STATS>
-__device__ __forceinline__ bool trace(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax, uint32_t self,
-                                      Stack& st, float* t_out, uint32_t* prim_out, PrimHit* hit_out, Stats* stats,
-                                      uint32_t* meta_out = nullptr) {
-  if (sc.width == 4)
-    return trace4<STATS>(sc, o, d, time, tmin, tmax, self, st, t_out, prim_out, hit_out, stats, meta_out);
-  return trace2<STATS>(sc, o, d, time, tmin, tmax, self, st, t_out, prim_out, hit_out, stats, meta_out);
+__device__ __forceinline__ bool trace(const DScene& sc, f3 o, f3 d, float time, float tmin, float tmax, Stack& st,
+                                      float* t_out, uint32_t* prim_out, PrimHit* hit_out, Stats* stats) {
+  if (sc.width == 4) return trace4<STATS>(sc, o, d, time, tmin, tmax, st, t_out, prim_out, hit_out, stats);
+  return trace2<STATS>(sc, o, d, time, tmin, tmax, st, t_out, prim_out, hit_out, stats);
 }
 
 // ---- resumable walk -----------------------------------------------------------
@@ -850,13 +825,14 @@ __device__ __forceinline__ bool trace(const DScene& sc, f3 o, f3 d, float time, 
 // lanes do. tmin is SHADOW_ACNE and the interval starts unbounded.
 constexpr uint32_t kNoNode = 0xffffffffu;  // walk over (has the leaf bit; no leaf has this index)
 constexpr uint32_t kNoPrim = 0xffffffffu;
+constexpr uint32_t kNoSelf = 0xffffffffu;  // a camera ray starts on no primitive
 struct Walk {
   f3 o, d;
   float inv[3];
   float rdd;     // 1 / |d|^2
   float time, closest;
   uint32_t cur;  // node, GT_LEAF_BIT | primitive, or kNoNode
-  uint32_t self, best;
+  uint32_t self, best;  // primitives (leaf order): where the ray starts (or kNoSelf), the closest hit (or kNoPrim)
 };
 // The scene's part that the steps read, with pointers known to be global.
 struct WalkScene {
@@ -945,6 +921,13 @@ __device__ __forceinline__ void walk_inner(const WalkScene& sc, Walk& w, Stack& 
 }
 // prim_test's decision and distance, with the tests of a kind in one straight line: a wave takes
 // every path some lane needs, so early exits save nothing, and sphere_hit's quotients share 1 / |d|^2.
+//
+// self: the ray starts on this primitive. A ray leaving a plane cannot meet it again (the reference's t
+// is 0 up to rounding, below t_min). On a sphere one root is then 0 in exact arithmetic and the other
+// 2h/a, so it is met again only by a ray heading inward, at the far root. FP32 cannot place the origin
+// on a large sphere within t_min (on the 1000-radius ground sphere a coordinate's ulp is 6e-5 and the
+// near root's error grows as 1/cos at grazing angles), so the near root is skipped by this rule, not
+// compared with t_min: the decision the reference's f64 arithmetic makes.
 __device__ __forceinline__ bool walk_test(const GPrim* __restrict__ prims, uint32_t k, const Walk& w, float* t_out,
                                           uint32_t* meta_out) {
   const float4* rec = reinterpret_cast<const float4*>(prims + k);
@@ -952,7 +935,7 @@ __device__ __forceinline__ bool walk_test(const GPrim* __restrict__ prims, uint3
   const uint32_t meta = meta_of(p0);
   *meta_out = meta;
   const uint32_t kind = (meta >> GT_KIND_SHIFT) & GT_KIND_MASK;
-  const bool self = k == w.self;  // the ray starts on this primitive: a plane is not met again
+  const bool self = k == w.self;
   const float tmin = SHADOW_ACNE, tmax = w.closest;
   if (kind == GK_TRIANGLE) {  // tri_hit
     const float4 p2 = rec[2];

@@ -221,10 +221,6 @@ __device__ __forceinline__ void wave_count(unsigned long long* dst, uint32_t v) 
 __device__ __forceinline__ unsigned long long* count_slot(const Queues& q, uint32_t bounce, int k) {
   return q.tally + 1 + 4 * bounce + k;
 }
-__device__ __forceinline__ uint32_t node_fetches(const Stats& s, uint32_t width) {
-  // every internal node fetched tests `width` child boxes; the root box test is not a fetch
-  return (s.node_tests - 1) / width;
-}
 
 // Shading category of a primitive's material.
 __device__ __forceinline__ uint32_t category_of(uint32_t meta) {
@@ -972,7 +968,7 @@ __global__ void k_aov(Frame f, Queues q, float* albedo, float* normal) {
       uint32_t prim;
       camera_ray(f.cam, x, y, s, rng, &o, &d, &time);
       PrimHit ph{0.f, 0.f, 0.f};
-      if (trace<false>(f.scene, o, d, time, SHADOW_ACNE, INF, kNoSelf, st, &t, &prim, &ph, nullptr)) {
+      if (trace<false>(f.scene, o, d, time, SHADOW_ACNE, INF, st, &t, &prim, &ph, nullptr)) {
         refine_hit(f.scene.prims, prim, o, d, time, SHADOW_ACNE, &ph);
         t = ph.t;
         f3 p = o + t * d;
@@ -1010,7 +1006,7 @@ __global__ void k_intersect(Frame f, Queues q, const float4* __restrict__ rays, 
     uint32_t prim = 0;
     PrimHit ph{0.f, 0.f, 0.f};
     Stats s{0, 0, 0, 0, 0, 0};
-    bool hit = trace<STATS>(f.scene, o, d, o4.w, tmin, d4.w, kNoSelf, st, &t, &prim, &ph, &s);
+    bool hit = trace<STATS>(f.scene, o, d, o4.w, tmin, d4.w, st, &t, &prim, &ph, &s);
     if (hit) {
       refine_hit(f.scene.prims, prim, o, d, o4.w, tmin, &ph);  // the chosen primitive's t, u, v in FP64
       t = ph.t;

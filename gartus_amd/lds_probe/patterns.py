@@ -7,9 +7,9 @@ Two kinds of entries, one probe dispatch each:
   lanes are served in the same pass, so the list of b that conflict with a
   gives the lane grouping of each access width;
 - the LDS accesses of the denoiser's kernels, as they are laid out now and
-  as they were before (the MFMA operand reads of k_conv and k_conv_pipe, the
-  weight gradient's operand reads and its staging writes), every read of one
-  chunk or tile in one dispatch.
+  as they were before (the MFMA operand reads of k_conv, the weight
+  gradient's operand reads and its staging writes), every read of one chunk
+  or tile in one dispatch.
 """
 import json
 import struct
@@ -75,10 +75,6 @@ def operand_reads(G, NT, mirror, row_bytes, swz, weights_base):
 def kernel_layouts():
     none = lambda p: 0
     layouts = [
-        ("k_conv_pipe 16-channel chunks, now: 32-byte pixels", 1, 32, none),
-        ("k_conv_pipe 16-channel chunks, before: pieces ^ (p >> 3) & 1", 1, 32, lambda p: (p >> 3) & 1),
-        ("k_conv_pipe 32-channel chunks, now: pieces ^ (p >> 1) & 3", 2, 64, lambda p: (p >> 1) & 3),
-        ("k_conv_pipe 32-channel chunks, before: pieces ^ (p >> 2) & 3", 2, 64, lambda p: (p >> 2) & 3),
         ("k_conv 32-channel chunks, now: 64-byte rows, pieces ^ (p >> 1) & 3", 2, 64, lambda p: (p >> 1) & 3),
         ("k_conv 16-channel chunks, now: 64-byte rows, pieces ^ (p >> 1) & 3", 1, 64, lambda p: (p >> 1) & 3),
         ("k_conv 32-channel chunks, before: 80-byte rows", 2, 80, none),
