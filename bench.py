@@ -331,6 +331,11 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
     def ndisp(c, kernels, ctr):
         return sum(len(c.get(k, {}).get(ctr, [])) for k in kernels)
 
+    def issue_share(insts, gui):
+        """Of the SIMDs' issue cycles: an instruction of 64 lanes takes 4 of one of the 1024 SIMDs; the busy
+        cycles are summed over the 8 XCDs."""
+        return 4.0 * insts / (1024 * gui / 8) if gui else None
+
     def row(kernels):
         n = ndisp(fe, kernels, "FETCH_SIZE")
         rd = tot(fe, kernels, "FETCH_SIZE") * f_fetch * 1024 / n
@@ -342,7 +347,8 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
                 "l2_hit_rate": hit / (hit + miss) if hit + miss else None,
                 "wave_wait_frac": tot(sq, kernels, "SQ_WAIT_ANY") / wave if wave else None,
                 "valu_busy_frac": valu / wave if wave else None,
-                "valu_lane_util": tot(sq, kernels, "SQ_THREAD_CYCLES_VALU") / (64.0 * valu) if valu else None}
+                "valu_lane_util": tot(sq, kernels, "SQ_THREAD_CYCLES_VALU") / (64.0 * valu) if valu else None,
+                "valu_issue_frac": issue_share(tot(sq, kernels, "SQ_INSTS_VALU"), tot(sq, kernels, "GRBM_GUI_ACTIVE"))}
 
     # the timed kernels: counting instantiations (first template argument true) left out
     timed = {k for k in fe if k.startswith(("k_extend<false", "k_shade", "k_connect<false", "k_accumulate"))}
@@ -380,7 +386,7 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
     traffic_file = dest / TRAFFIC_FILE.name
     rec = json.loads(traffic_file.read_text()) if traffic_file.exists() else {}
     rec[workload] = {
-        "kernel": "k_extend<false, *, *> (bounce 0 and later bounces)",
+        "kernel": "k_extend<false, *, *, *> (bounce 0 and later bounces)",
         "kernel_sources_sha16": kernel_sources_sha(),
         "bytes_per_launch": round(bytes_per_launch),
         "fetch_factor": round(f_fetch, 4),
@@ -389,6 +395,7 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
         "wave_wait_frac": round(e["wave_wait_frac"], 4),
         "valu_busy_frac": round(e["valu_busy_frac"], 4),
         "valu_lane_util": round(e["valu_lane_util"], 4),
+        "valu_issue_frac": None if e["valu_issue_frac"] is None else round(e["valu_issue_frac"], 4),
         "rocprof_avg_launch_us": round(avg_us, 1),
         "source": f"profiles/{workload}_counters.md",
         "commands": _profile_commands(workload),
@@ -409,11 +416,12 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
               "Infinity Cache serves are counted too: an upper bound on HBM reads.", "",
               "Per dispatch means over the counter runs' timed renders (the counting render left out). Wait = "
               "SQ_WAIT_ANY / SQ_WAVE_CYCLES (share of wave time waiting on anything, mostly memory); VALU busy = "
-              "SQ_ACTIVE_INST_VALU / SQ_WAVE_CYCLES; lane use = SQ_THREAD_CYCLES_VALU / (64 x "
+              "SQ_ACTIVE_INST_VALU / SQ_WAVE_CYCLES, of one wave's cycles; VALU issue = 4 x SQ_INSTS_VALU / (1024 x "
+              "GRBM_GUI_ACTIVE / 8), of the SIMDs' cycles; lane use = SQ_THREAD_CYCLES_VALU / (64 x "
               "SQ_ACTIVE_INST_VALU), the active-lane share of VALU issue (divergence). Durations: mean of the "
               "trace run's dispatches (all renders, from run_kernel_stats.csv).", "",
               "| kernel | dispatches | mean us | HBM read MB | HBM write MB | GB/s | L2 hit | wait | VALU busy | "
-              "lane use |", "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
+              "VALU issue | lane use |", "|---|---:|---:|---:|---:|---:|---:|---:|---:|---:|---:|"]
     order = sorted(timed, key=lambda k: -float(stats.get(k, {}).get("TotalDurationNs", 0) or 0))
     for k in order:
         r = row([k])
@@ -422,7 +430,7 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
         f3 = (lambda v: "-" if v is None else f"{v:.3f}")
         lines.append(f"| {k} | {r['dispatches']} | {us:.1f} | {r['read_bytes'] / 1e6:.1f} | "
                      f"{r['write_bytes'] / 1e6:.1f} | {gbs:.0f} | {f3(r['l2_hit_rate'])} | "
-                     f"{f3(r['wave_wait_frac'])} | {f3(r['valu_busy_frac'])} | {f3(r['valu_lane_util'])} |")
+                     f"{f3(r['wave_wait_frac'])} | {f3(r['valu_busy_frac'])} | {f3(r['valu_issue_frac'])} | {f3(r['valu_lane_util'])} |")
     lines += ["", "## The roofline kernel (extend)", "",
               f"- HBM traffic per launch: {bytes_per_launch:,.0f} bytes (reads {e['read_bytes']:,.0f}, writes "
               f"{e['write_bytes']:,.0f}), over {e['dispatches']} dispatches; L2 hit rate {e['l2_hit_rate']:.3f}.",
@@ -442,8 +450,9 @@ def record_profile(out: Path, workload: str, calibrate_mib: int = 1024, dest: Pa
          "    " + _profile_commands(workload)[3], "",
          f"The run renders the workload {renders + 1} times: a statistics render, {warmup} warm-up, {steps} timed "
          "steps and a traversal-counting render (the instantiations whose first template argument is true). "
-         "k_extend<COUNT, MULTI, CAMERA>, k_connect<COUNT, MULTI>, k_shade<MULTI, CAMERA>; MULTI is the batched "
-         "(frame-table) form, CAMERA the bounce of the camera rays. Durations in microseconds, from "
+         "k_extend<COUNT, MULTI, CAMERA, WIDE>, k_connect<COUNT, MULTI, WIDE, KIND>, k_shade<MULTI, CAMERA>; MULTI is "
+         "the batched (frame-table) form, CAMERA the bounce of the camera rays, WIDE four-wide nodes, KIND 0 light "
+         "and 1 environment shadow rays. Durations in microseconds, from "
          "run_kernel_stats.csv.", "", "| kernel | calls | total us | average us | % |", "|---|---:|---:|---:|---:|"]
     for k, r in sorted(stats.items(), key=lambda kv: -float(kv[1]["TotalDurationNs"])):
         t.append(f"| {k} | {r['Calls']} | {float(r['TotalDurationNs']) * 1e-3:.1f} | {float(r['AverageNs']) * 1e-3:.2f} "
@@ -535,6 +544,7 @@ def roofline_record(measured: dict, traffic, hbm_gbs, algorithmic_gbs: float, al
         "wave_wait_frac": measured.get("wave_wait_frac"),
         "valu_busy_frac": measured.get("valu_busy_frac"),
         "valu_lane_util": measured.get("valu_lane_util"),
+        "valu_issue_frac": measured.get("valu_issue_frac"),
         "counters_source": measured.get("source"),
     })
     rec["limiter"] = limiter(rec)
@@ -544,16 +554,20 @@ def roofline_record(measured: dict, traffic, hbm_gbs, algorithmic_gbs: float, al
 def limiter(rec: dict) -> str | None:
     """What the counters say bounds the kernel: HBM bandwidth when the
     measured traffic runs near peak; otherwise, when waves spend most of
-    their cycles waiting with little VALU issue, the latency of dependent
-    memory fetches; None without counters."""
+    their cycles waiting with little VALU issue (of a wave's cycles, and of
+    the SIMDs'), the latency of dependent memory fetches; None without counters."""
     wait, busy = rec.get("wave_wait_frac"), rec.get("valu_busy_frac")
+    issue = rec.get("valu_issue_frac")
     if rec.get("traffic") is None or wait is None or busy is None:
         return None
     if rec["frac"] >= 0.7:
         return "HBM bandwidth"
-    if wait >= 0.5 and busy < 0.25:
+    if wait >= 0.5 and busy < 0.25 and (issue is None or issue < 0.4):
         return (f"latency of dependent memory fetches: HBM at {rec['frac']:.2f} of peak, waves waiting "
                 f"{100 * wait:.0f}% of their cycles, VALU issuing {100 * busy:.0f}%")
+    if issue is not None:
+        return (f"mixed: HBM at {rec['frac']:.2f} of peak, VALU issuing {100 * issue:.0f}% of the SIMDs' cycles, "
+                f"waves waiting {100 * wait:.0f}% of theirs")
     return f"mixed: HBM at {rec['frac']:.2f} of peak, waves waiting {100 * wait:.0f}%, VALU {100 * busy:.0f}%"
 
 

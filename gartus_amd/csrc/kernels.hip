@@ -235,7 +235,7 @@ __device__ __forceinline__ uint32_t category_of(uint32_t meta) {
 }
 
 // ---- traversal with refill ---------------------------------------------------
-// What bounds the traversal kernels is the vector ALU: before, its instructions
+// What bounded the traversal kernels was the vector ALU: its instructions
 // filled 70 to 98 % of a SIMD's cycles on the 1080p GGX/environment frame and
 // the 720p terrain, with 21 to 40 % of their lanes at work, because the rays of
 // a wave differ widely in length and wait for the longest. So the walk of
@@ -246,10 +246,13 @@ __device__ __forceinline__ uint32_t category_of(uint32_t meta) {
 // carried state is only what a step changes (carrying the whole ray around one
 // common loop cost 32 moves a step); everything else is read from the kernel's
 // arguments when it is needed. Measured against one ray per lane at a time, on
-// one MI355X: 720p terrain 16.2 -> 13.7 ms, 1080p GGX/environment 14.4 -> 13.1 ms,
-// 12 small scenes in one batch 8.3 -> 5.3 ms (also for the scene pointers no
+// one MI355X: 720p terrain 16.2 -> 13.7 ms, 1080p GGX/environment 14.1 -> 12.9 ms,
+// 12 small scenes in one batch 7.6 -> 5.1 ms (also for the scene pointers no
 // longer being generic, whose loads were flat instructions). Camera rays are
-// coherent and as long as their neighbours: they take no refill.
+// coherent and as long as their neighbours: they take no refill. Now camera rays
+// fill 96 % of the issue cycles, with 47 % (terrain) and 83 % (1080p frame) of
+// the lanes; the later bounces fill 44 and 60 %, with 43 and 60 %, and wait on
+// node fetches for the rest.
 constexpr uint32_t kRing = 128;                   // entries of a wave's ring: at most 63 + 64 are held
 constexpr uint32_t kRingWords = 2 * kRing;        // extend: finished hits, finished misses
 constexpr uint32_t kNoPath = 0xffffffffu;

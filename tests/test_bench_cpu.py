@@ -127,4 +127,6 @@ def test_limiter_reads_the_counters():
     assert bench.limiter(dict(base, frac=0.8)) == "HBM bandwidth"
     assert bench.limiter(dict(base, traffic=None)) is None
     assert bench.limiter(dict(base, wave_wait_frac=0.2)).startswith("mixed")
+    assert bench.limiter(dict(base, valu_issue_frac=0.3)).startswith("latency of dependent memory fetches")
+    assert "VALU issuing 68%" in bench.limiter(dict(base, valu_issue_frac=0.68))  # eight waves share a SIMD
 
