@@ -283,7 +283,7 @@ PROFILE_PASSES = {
     "fetch": "FETCH_SIZE",
     "write": "WRITE_SIZE TCC_HIT_sum TCC_MISS_sum",
 }
-TUNING_ARGS = {"batch64": "--block 64 --bvh-width 4 --max-paths 67108864"}
+TUNING_ARGS = {"batch64": "--block 64 --bvh-width 2 --max-paths 67108864"}  # what the autotuner picks
 
 
 def _profile_commands(workload: str) -> list[str]:
